@@ -2464,42 +2464,6 @@ extern "C" int sf_gemm(const sf_gemm_desc* d, void* stream) {
 }
 
 // ---------------------------------------------------------------------------
-// Column sums (bias gradient): a workgroup owns 64 columns; its 4 waves take
-// interleaved rows and fold their partial sums in LDS in a fixed order.
-// ---------------------------------------------------------------------------
-namespace sf {
-namespace {
-__global__ void __launch_bounds__(256) column_sum_kernel(const void* __restrict__ A, int a_dtype, int64_t rows,
-                                                         int64_t cols, void* __restrict__ out, int out_dtype) {
-  __shared__ float part[4][64];
-  const int c = threadIdx.x & 63, rg = threadIdx.x >> 6;
-  const int64_t col = blockIdx.x * 64ll + c;
-  float s = 0.0f;
-  if (col < cols)
-    for (int64_t r = rg; r < rows; r += 4) s += load_as_f32(A, r * cols + col, a_dtype);
-  part[rg][c] = s;
-  __syncthreads();
-  if (rg == 0 && col < cols)
-    store_from_f32(out, col, out_dtype, ((part[0][c] + part[1][c]) + part[2][c]) + part[3][c]);
-}
-}  // namespace
-}  // namespace sf
-
-extern "C" int sf_column_sum(const void* A, int a_dtype, int64_t rows, int64_t cols, void* out, int out_dtype,
-                             void* stream) {
-  SF_CHECK_ARG(rows >= 0 && cols >= 0, "negative shape");
-  SF_CHECK_ARG((a_dtype == SF_DTYPE_F32 || a_dtype == SF_DTYPE_BF16) &&
-                   (out_dtype == SF_DTYPE_F32 || out_dtype == SF_DTYPE_BF16),
-               "bad dtype");
-  if (cols == 0) return SF_OK;
-  SF_CHECK_ARG(out && (rows == 0 || A), "null tensor");
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(column_sum_kernel, dim3(static_cast<unsigned>(ceil_div(cols, 64))), dim3(256), 0, st, A, a_dtype,
-                     rows, cols, out, out_dtype);
-  return launch_status("sf_column_sum");
-}
-
-// ---------------------------------------------------------------------------
 // 2:4 packed weights and the sparse-MFMA forward (finalized / inference
 // models: legacy/main_llama.py:2499-2568 hardens the masks and multiplies
 // them into the weights; legacy/eval_wiki_ppl.py:548-651 then runs the plain
