@@ -57,11 +57,15 @@ __host__ __device__ __forceinline__ float bf16_to_f32(uint16_t h) {
 }
 
 __host__ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));  // one v_cvt_pk_bf16_f32 (a NaN stays a quiet NaN)
+#else
   uint32_t u;
   memcpy(&u, &f, 4);
   if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x0040u);  // quiet NaN
   u += 0x7fffu + ((u >> 16) & 1u);
   return static_cast<uint16_t>(u >> 16);
+#endif
 }
 
 // Round an f32 to the nearest bf16 and return it as f32.

@@ -178,6 +178,33 @@ __device__ __forceinline__ void sqrt_rn4(const float x[4], float r[4]) {
   }
 }
 
+// |W| / sqrt(H + eps) of a group when W and H are both bf16 (so every op rounds to bf16), without the
+// corrections that make the f32 root and quotient exact: hp (the bf16 sum) has an 8-bit significand, so
+// sqrt(hp) is never closer to a bf16 rounding boundary (a 9-bit significand m) than |hp - m^2| / (2 m) >=
+// 2^-19 of itself, and the quotient of two bf16 values never closer than 2^-18 to one (w = m sq has no
+// solution in 8 bits for an odd 9-bit m); the hardware root (1 ulp of f32) and w * v_rcp_f32 (at most 2)
+// therefore round to the same bf16 as the correctly rounded f32 results do (tests/test_bf16_score_rounding.py
+// goes through every significand).  Zeros, infinities, NaN and results near the ends of the exponent range
+// fail one range test per group and take the exact path.
+__device__ __forceinline__ void ratio_scores_bf16(const float w[4], const float h[4], float eps, float sc[4]) {
+  constexpr uint32_t lo = 0x0D800000u, width = 0x72000000u - 0x0D800000u;  // 2^-100 .. 2^101
+  uint32_t u = 0;
+  float hp[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    hp[j] = round_bf16(h[j] + eps);
+    const float q = fabsf(w[j]) * __builtin_amdgcn_rcpf(round_bf16(__builtin_amdgcn_sqrtf(hp[j])));
+    const uint32_t a = __float_as_uint(hp[j]) - lo, b = __float_as_uint(q) - lo;
+    u = a > u ? a : u;
+    u = b > u ? b : u;
+    sc[j] = round_bf16(q);
+  }
+  if (__builtin_expect(u >= width, 0)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) sc[j] = round_bf16(fabsf(w[j]) / round_bf16(sqrtf(hp[j])));
+  }
+}
+
 template <int WD, int HD>
 __device__ __forceinline__ float score_of(const ScoreSpec& s, float w, float h, float a) {
   constexpr int PWH = (WD == SF_DTYPE_F32 || HD == SF_DTYPE_F32) ? SF_DTYPE_F32 : SF_DTYPE_BF16;
@@ -244,13 +271,16 @@ template <int WD, int HD>
 __device__ __forceinline__ void scores_of_ops(const ScoreSpec& s, const GroupOps& o, const Group& g, float sc[4]) {
   const float *w = o.w, *h = o.h, *a = o.a;
   if (s.metric == SF_METRIC_HESSIAN_RATIO && g.n == 4) {  // |W| / sqrt(H + eps), the sqrt range test per group
-    constexpr int PWH = (WD == SF_DTYPE_F32 || HD == SF_DTYPE_F32) ? SF_DTYPE_F32 : SF_DTYPE_BF16;
-    float hp[4], sq[4];
+    if constexpr (WD == SF_DTYPE_BF16 && HD == SF_DTYPE_BF16) {
+      ratio_scores_bf16(w, h, s.eps, sc);
+    } else {  // the quotient is an f32 score
+      float hp[4], sq[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) hp[j] = rndc<HD>(h[j] + s.eps);
-    sqrt_rn4(hp, sq);
+      for (int j = 0; j < 4; ++j) hp[j] = rndc<HD>(h[j] + s.eps);
+      sqrt_rn4(hp, sq);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) sc[j] = rndc<PWH>(fabsf(w[j]) / rndc<HD>(sq[j]));
+      for (int j = 0; j < 4; ++j) sc[j] = fabsf(w[j]) / rndc<HD>(sq[j]);
+    }
     return;
   }
   // one switch per group, the element loop inside each case
@@ -411,7 +441,18 @@ __global__ void __launch_bounds__(kBlock) flip_count_kernel(const void* __restri
 // Score statistics: per-workgroup f64 partial sums, then one workgroup folds
 // them in a fixed order (deterministic for a fixed grid).
 // ---------------------------------------------------------------------------
-constexpr int kStatsGrid = 4096;
+constexpr int kStatsGrid = 4096;  // most workgroups (and partials) of a layer
+
+// Workgroups of a layer's statistics pass: 8 groups per thread, so that a workgroup's set-up and its f64
+// reduction (two barriers) are spread over 8 rounds of loads, but no fewer than fill the GPU once.  With the
+// fixed 4096 a 2048 x 2048 layer gave every thread one group: 28 bf16 layers of a 1.1B model's shapes
+// 482 us, 8 groups a thread 229 us (with the bf16 scores below).
+__host__ __device__ __forceinline__ int stats_blocks(int64_t groups) {
+  int64_t b = ceil_div(groups, 8 * kBlock);
+  const int64_t fill = ceil_div(groups, kBlock) < 256 ? ceil_div(groups, kBlock) : 256;
+  b = b < fill ? fill : b;
+  return static_cast<int>(b > kStatsGrid ? kStatsGrid : (b < 1 ? 1 : b));
+}
 
 __device__ __forceinline__ void block_sum2_f64(double a, double b, double* out_a, double* out_b) {
   __shared__ double ra[kBlock / 64], rb[kBlock / 64];
@@ -436,7 +477,7 @@ __device__ __forceinline__ void block_sum2_f64(double a, double b, double* out_a
   }
 }
 
-// Partial sums of workgroup `blk` of the kStatsGrid-workgroup grid over one
+// Partial sums of workgroup `blk` of the stats_blocks(groups) workgroups over one
 // layer.  VEC: every group full and vector-loadable (as in update_mask_kernel).
 // RATIO: the metric is hessian_ratio (|W| / sqrt(H + eps), no aux operand), fixed at compile time.
 // NT: W and H through non-temporal loads (the batched arena pass).
@@ -463,7 +504,7 @@ __device__ __forceinline__ void stats_partial_block(const ScoreSpec& s_in, const
         sq += d * d;
       }
   };
-  GroupWalk w(groups, cols, gpr, blk, kStatsGrid);
+  GroupWalk w(groups, cols, gpr, blk, stats_blocks(groups));
   if constexpr (VEC) {
     // two groups per round, both loaded before either is used (the sums keep the walk's order)
     while (w.live()) {
@@ -504,7 +545,7 @@ __global__ void __launch_bounds__(kBlock) stats_partial_kernel(ScoreSpec s, cons
   stats_partial_block<WD, HD, VEC, RATIO>(s, W, H, aux, cols, groups, gpr, vec, partial, blockIdx.x);
 }
 
-// Fold of one layer's kStatsGrid partials by one workgroup, in a fixed order.
+// Fold of one layer's partials by one workgroup, in a fixed order.
 __device__ __forceinline__ void stats_final_block(const double* __restrict__ partial, int nparts, int64_t n,
                                                   float* stats) {
   // 8 partials per thread and round, their loads issued together: the partials
@@ -1087,12 +1128,14 @@ __device__ __forceinline__ int flips_of(const float a[4], const float b[4], cons
   return __popc((hard_bits(a, g, kind, n) ^ hard_bits(b, g, kind, n)) & ((1u << g.n) - 1u));
 }
 
-// Specialisations of the fused update for the configurations training runs
-// spend their time in: kFastPlain = hessian_ratio scores, unstructured gate,
+// Specialisations of the fused update (all-f32 scores and mask, or W, H, scores and mask all bf16) for the
+// configurations training runs spend their time in: kFastPlain = hessian_ratio scores, unstructured gate,
 // no penalty, binarisation, frozen flags, freezing or structural mix, 2:4 flip
 // count; kFastNm24 = the same with the nm_2_4 penalty.  The spec's fields are
 // fixed to those values, so the compiler drops every other branch (the
-// arithmetic is the generic path's, operation for operation).
+// arithmetic is the generic path's, operation for operation).  Bound by VALU
+// issue in bf16 (8 B but about 90 instructions per element): 28 bf16 layers of
+// a 1.1B model's shapes (205 M weights) 961 us on the generic kernel, 551 us.
 constexpr int kFastNone = 0, kFastPlain = 1, kFastNm24 = 2;
 
 template <int FAST>
@@ -1217,7 +1260,7 @@ __global__ void __launch_bounds__(kBlock) update_mask_kernel(UpdateSpec us, cons
 // Multi-layer mask update: the score statistics, tau selection and fused
 // update of up to kMultiLayers layers that share every parameter but their
 // shape, as a handful of launches.  Each layer runs exactly the workgroup
-// grid its single-layer launch would (the statistics' kStatsGrid partials
+// grid its single-layer launch would (the statistics' partials
 // fold in the same order, the update walks the same groups), laid end to end
 // in one grid, so every output equals the single-layer entry points' bit for
 // bit.  The layer table travels in the kernel arguments.
@@ -1259,7 +1302,8 @@ __device__ __forceinline__ int multi_layer_of(const MultiArgs& a, int b) {
   return l;
 }
 
-// Statistics partials: kStatsGrid workgroups per layer, layer = blockIdx.x / kStatsGrid.
+// Statistics partials: kStatsGrid workgroup ids per layer (layer = id / kStatsGrid), of which the first
+// stats_blocks(groups) work.
 // The first n * gather workgroups gather the layers' tau samples (gather per
 // layer; 0 when the tau stage runs on its own), the rest are the statistics
 // grids.  The gather's random reads go first and overlap the statistics pass,
@@ -1277,6 +1321,7 @@ __global__ void __launch_bounds__(kBlock) stats_partial_multi_kernel(MultiArgs a
   const int l = b / kStatsGrid, blk = b - l * kStatsGrid;
   const MultiLayer& L = a.l[l];
   const int64_t gpr = ceil_div(L.cols, 4);
+  if (blk >= stats_blocks(L.rows * gpr)) return;  // the whole workgroup
   stats_partial_block<WD, HD, VEC, RATIO, true>(a.us.gs.s, L.W, L.H, L.aux, L.cols, L.rows * gpr, gpr, L.vec != 0,
                                           partial + (int64_t)l * 2 * kStatsGrid, blk);
 }
@@ -1284,7 +1329,7 @@ __global__ void __launch_bounds__(kBlock) stats_partial_multi_kernel(MultiArgs a
 // ---------------------------------------------------------------------------
 // Statistics with the tau sample folded in (batched update, every layer's
 // groups vector-loadable).  Round r of statistics workgroup b covers the
-// 1024 elements [1024 (b + r kStatsGrid), +1024), each wave a 256-element
+// 1024 elements [1024 (b + r stats_blocks), +1024), each wave a 256-element
 // sub-window of them (64 lanes x one group), so every element is scored
 // exactly once per pass.  When a layer's sample is in non-decreasing index
 // order, the samples that fall in sub-window v are the positions
@@ -1366,7 +1411,7 @@ __device__ __forceinline__ void stats_fold_block(const ScoreSpec& s_in, const Mu
   // raw scores of the wave's two sub-windows of an iteration, double-buffered: [wave][parity][round][element]
   __shared__ __align__(16) float win[kBlock / 64][2][2][256];
   float(*mine)[2][256] = win[wave];
-  const int64_t stride = (int64_t)kStatsGrid * kBlock;
+  const int64_t stride = (int64_t)stats_blocks(groups) * kBlock;
   double sum = 0.0, sq = 0.0;
   // The previous iteration's samples, resolved in one pass: lane l serves sample (l % 32) of sub-window
   // l / 32 (rounds 0 and 1), so its range, element base and first index are this lane's.
@@ -1462,12 +1507,15 @@ template <int WD, int HD>
 __global__ void __launch_bounds__(kBlock) stats_fold_multi_kernel(MultiArgs a, double* partial, uint32_t* keys,
                                                                   const int32_t* wstart) {
   const int l = blockIdx.x / kStatsGrid, blk = blockIdx.x - l * kStatsGrid;
+  if (blk >= stats_blocks(a.l[l].rows * (a.l[l].cols >> 2))) return;  // the whole workgroup
   stats_fold_block<WD, HD>(a.us.gs.s, a.l[l], wstart, keys, partial + (int64_t)l * 2 * kStatsGrid, blk);
 }
 
 __global__ void __launch_bounds__(kBlock) stats_final_multi_kernel(MultiArgs a, const double* partial) {
   const int l = blockIdx.x;
-  stats_final_block(partial + (int64_t)l * 2 * kStatsGrid, kStatsGrid, a.l[l].rows * a.l[l].cols, a.l[l].stats);
+  const int64_t groups = a.l[l].rows * ceil_div(a.l[l].cols, 4);
+  stats_final_block(partial + (int64_t)l * 2 * kStatsGrid, stats_blocks(groups), a.l[l].rows * a.l[l].cols,
+                    a.l[l].stats);
 }
 
 // tau: grid (x, layer); each layer's gather strides over gridDim.x workgroups,
@@ -1736,17 +1784,17 @@ extern "C" int sf_score_stats(const sf_mask_params* p, const void* W, int w_dtyp
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (vec && p->metric == SF_METRIC_HESSIAN_RATIO)
     SF_DISPATCH_WH(w_dtype, h_dtype,
-                   stats_partial_kernel<WD_, HD_, true, true><<<kStatsGrid, kBlock, 0, st>>>(
+                   stats_partial_kernel<WD_, HD_, true, true><<<stats_blocks(groups), kBlock, 0, st>>>(
                        s, W, H, aux, p->cols, groups, gpr, vec, partial));
   else if (vec)
     SF_DISPATCH_WH(w_dtype, h_dtype,
-                   stats_partial_kernel<WD_, HD_, true, false><<<kStatsGrid, kBlock, 0, st>>>(
+                   stats_partial_kernel<WD_, HD_, true, false><<<stats_blocks(groups), kBlock, 0, st>>>(
                        s, W, H, aux, p->cols, groups, gpr, vec, partial));
   else
     SF_DISPATCH_WH(w_dtype, h_dtype,
-                   stats_partial_kernel<WD_, HD_, false, false><<<kStatsGrid, kBlock, 0, st>>>(
+                   stats_partial_kernel<WD_, HD_, false, false><<<stats_blocks(groups), kBlock, 0, st>>>(
                        s, W, H, aux, p->cols, groups, gpr, vec, partial));
-  stats_final_kernel<<<1, kBlock, 0, st>>>(partial, kStatsGrid, n, stats_out);
+  stats_final_kernel<<<1, kBlock, 0, st>>>(partial, stats_blocks(groups), n, stats_out);
   return launch_status("sf_score_stats");
 }
 
@@ -2055,10 +2103,19 @@ extern "C" int sf_update_mask(const sf_mask_params* p, const void* W, int w_dtyp
     else
       SF_LAUNCH_UPD(SF_DTYPE_F32, SF_DTYPE_BF16);
   } else {
-    if (sf32)
+    const bool b16 = w_dtype == SF_DTYPE_BF16 && h_dtype == SF_DTYPE_BF16 && !sf32;
+#define SF_LAUNCH_UPD_B16(FAST)                                                                             \
+  update_mask_kernel<SF_DTYPE_BF16, SF_DTYPE_BF16, SF_DTYPE_BF16, SF_DTYPE_BF16, true, FAST>                \
+      <<<grid, kBlock, 0, st>>>(us, W, H, aux, mask, frozen, stats, tau, p->cols, groups, gpr, vec, flips)
+    if (b16 && fk == kFastPlain)
+      SF_LAUNCH_UPD_B16(kFastPlain);
+    else if (b16 && fk == kFastNm24)
+      SF_LAUNCH_UPD_B16(kFastNm24);
+    else if (sf32)
       SF_LAUNCH_UPD(SF_DTYPE_BF16, SF_DTYPE_F32);
     else
       SF_LAUNCH_UPD(SF_DTYPE_BF16, SF_DTYPE_BF16);
+#undef SF_LAUNCH_UPD_B16
   }
 #undef SF_LAUNCH_UPD
 #undef SF_LAUNCH_UPD_V
@@ -2354,11 +2411,20 @@ extern "C" int sf_update_mask_multi(const sf_mask_params* p, float q, const sf_m
       else
         SF_LAUNCH_UPDM(SF_DTYPE_F32, SF_DTYPE_BF16);
     } else {
-      if (sf32)
+      const bool b16 = w_dtype == SF_DTYPE_BF16 && h_dtype == SF_DTYPE_BF16 && !sf32;
+#define SF_LAUNCH_UPDM_B16(FAST)                                                                       \
+  update_mask_multi_kernel<SF_DTYPE_BF16, SF_DTYPE_BF16, SF_DTYPE_BF16, SF_DTYPE_BF16, true, FAST>     \
+      <<<total, kBlock, 0, st>>>(a)
+      if (b16 && fk == kFastPlain)
+        SF_LAUNCH_UPDM_B16(kFastPlain);
+      else if (b16 && fk == kFastNm24)
+        SF_LAUNCH_UPDM_B16(kFastNm24);
+      else if (sf32)
         SF_LAUNCH_UPDM(SF_DTYPE_BF16, SF_DTYPE_F32);
       else
         SF_LAUNCH_UPDM(SF_DTYPE_BF16, SF_DTYPE_BF16);
     }
+#undef SF_LAUNCH_UPDM_B16
 #undef SF_LAUNCH_UPDM
 #undef SF_LAUNCH_UPDM_V
   };
