@@ -36,13 +36,10 @@
 #include <type_traits>
 
 #include "sf_common.hpp"
+#include "sf_mfma.hpp"
 
 namespace sf {
 namespace {
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
 constexpr int kThreads = 256;
 constexpr int kTileM = 256;
@@ -117,26 +114,6 @@ struct Tr<float> {
   static constexpr int DT = SF_DTYPE_F32;
 };
 
-// 16-byte vector as 4 dwords
-struct V4 {
-  uint32_t w[4];
-};
-
-__device__ __forceinline__ V4 ld16(const void* p) {
-  uint4 v = *reinterpret_cast<const uint4*>(p);
-  V4 r;
-  r.w[0] = v.x;
-  r.w[1] = v.y;
-  r.w[2] = v.z;
-  r.w[3] = v.w;
-  return r;
-}
-__device__ __forceinline__ V4 zero16() {
-  V4 r;
-  r.w[0] = r.w[1] = r.w[2] = r.w[3] = 0u;
-  return r;
-}
-
 // How B1 is masked while it is staged: not at all, by a multiplicative
 // effective mask in the element dtype (rounded as the reference does), or by
 // a byte and-mask (0x00 / 0xFF per element) for masks whose values are 0 or 1.
@@ -147,19 +124,6 @@ template <typename T, int MK>
 struct MaskWords {
   static constexpr int N = MK == kMaskMul ? 4 : (MK == kMaskByte ? (int)(16 / sizeof(T)) / 4 : 1);
 };
-
-// bf16 halves of a dword as f32, and the hardware round-to-nearest-even pack
-// (v_cvt_pk_bf16_f32) back to two bf16.
-__device__ __forceinline__ float lo_f(uint32_t w) { return __uint_as_float(w << 16); }
-__device__ __forceinline__ float hi_f(uint32_t w) { return __uint_as_float(w & 0xffff0000u); }
-__device__ __forceinline__ uint32_t pack2(float lo, float hi) {
-  bf16x2_t v;
-  v[0] = static_cast<__bf16>(lo);
-  v[1] = static_cast<__bf16>(hi);
-  return __builtin_bit_cast(uint32_t, v);
-}
-__device__ __forceinline__ float hround(float x) { return static_cast<float>(static_cast<__bf16>(x)); }
-__device__ __forceinline__ uint16_t hbits(float x) { return __builtin_bit_cast(uint16_t, static_cast<__bf16>(x)); }
 
 // Masked B vector.  Multiplicative mask, with the reference's rounding:
 // w = round(W * E), then round(w * s) when a weight-scaling factor is set.
@@ -237,26 +201,6 @@ struct Stage {
   V4 v[8];
   uint32_t e[MK == kMaskNone ? 1 : 8][MaskWords<T, MK>::N];
 };
-
-// Raw buffer loads: an SGPR resource holds the tensor base and its byte
-// extent; a lane offset at or past the extent reads zeros without touching
-// memory, which is how rows past M/N and k past K are padded.
-typedef __amdgpu_buffer_rsrc_t Rsrc;
-constexpr uint32_t kOob = 0x80000000u;  // a lane offset past every operand's extent (extents are < 2^31 bytes)
-
-__device__ __forceinline__ Rsrc make_rsrc(const void* base, int64_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes, 0x00020000);
-}
-__device__ __forceinline__ V4 bload(Rsrc r, uint32_t voff, uint32_t soff) {
-  typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-  u32x4 x = __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0);
-  V4 o;
-  o.w[0] = x[0];
-  o.w[1] = x[1];
-  o.w[2] = x[2];
-  o.w[3] = x[3];
-  return o;
-}
 
 // Per-thread load state of one operand for one tile and one K segment.
 //   K-contiguous (L == 0), element (r, k) at base[r * ld + k]: vector i of the
@@ -564,8 +508,6 @@ __device__ __forceinline__ void tile_coords(int64_t pid, int64_t tiles_m, int64_
   tm = first_m + r % gm;
   tn = r / gm;
 }
-
-__device__ __forceinline__ float load_elem(const void* p, int64_t i, int dtype) { return load_as_f32(p, i, dtype); }
 
 // Epilogue shared by the GEMM kernels: the 4 x 4 accumulator blocks of each
 // wave (its 128 x 128 share of the 256 x 256 tile) go to C, a split-K partial
@@ -2486,27 +2428,6 @@ extern "C" int sf_gemm(const sf_gemm_desc* d, void* stream) {
 namespace sf {
 namespace {
 
-typedef __bf16 bf16x16_t __attribute__((ext_vector_type(16)));
-
-struct Gemm24Args {
-  const void* x;       // [N = tokens, K] bf16, row pitch ldx
-  int64_t ldx;
-  const void* vals;    // M * K / 2 bf16, fragment order (vals_off)
-  const void* idx;     // u32 [M / 32][K / 64][2][32]
-  int64_t M, N, K;
-  const void* bias;    // [M] or null
-  int bias_dtype;
-  void* y;             // [N, M], row pitch ldy
-  int y_dtype;
-  int64_t ldy;
-  int64_t tiles_m, tiles_n;
-  int y_aligned;
-  // optional dense second segment y^T += A2 . B2^T: A2 [M, K2] and B2 [N, K2] bf16, K-contiguous
-  const void* A2;
-  const void* B2;
-  int64_t lda2, ldb2, K2;
-};
-
 constexpr int kEpi24Pitch = 68;  // f32 pitch of the transposed staging: 128 token rows x 64 out columns per wave
 constexpr uint32_t k24XBuf = 256u * kRowSw;  // one x stage: 256 token rows x 128 B
 
@@ -3010,11 +2931,12 @@ int launch_gemm24(const void* x, int64_t ldx, int64_t tokens, const void* vals, 
   g.lda2 = lds;
   g.ldb2 = ldz;
   g.K2 = rank > 0 ? rank : 0;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (gemm24_split_takes(g)) return launch_gemm24_split(g, st, what);
   static bool attr = false;
   if (int rc = set_smem(gemm24_kernel, smem24_bytes(), attr)) return rc;
   const int64_t tiles = g.tiles_m * g.tiles_n;
   SF_CHECK_ARG(tiles < (1ll << 31), "grid too large");
-  hipStream_t st = static_cast<hipStream_t>(stream);
   hipLaunchKernelGGL(gemm24_kernel, dim3(static_cast<unsigned>(tiles)), dim3(kThreads), smem24_bytes(), st, g);
   return launch_status(what);
 }
