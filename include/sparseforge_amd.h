@@ -561,6 +561,26 @@ int sf_from_heads(const void* g, int dtype, int64_t B, int64_t S, int64_t H, int
                   const float* sin, int rotate, int transposed, float scale, void* x_grad, void* stream);
 
 /*
+ * Causal softmax attention of the retrained model in bf16 with no S x S tensor
+ * in memory (HuggingFace's eager attention of the LlamaForCausalLM that
+ * legacy/model_llama.py:39-55 wraps, and its first derivative).  q, k, v, out
+ * and the gradients are [B, S, H, D] (the projections' rows), D 64 or 128, each
+ * tensor below 2 GiB per batch entry and 16-byte aligned.
+ *   forward:  q_rot, k_rot = rot(q), rot(k) (sf_to_heads' rotation, kept for the
+ *             backward), out = softmax(scale q_rot k_rot^T, causal) v with the
+ *             scores and sums in f32, lse [B * H, S] = the base-2 logarithm of
+ *             every row's sum of 2^(scale log2(e) score)
+ *   backward: dq, dk (through the rotation's adjoint) and dv from grad_out;
+ *             delta [B * H, S] f32 is scratch
+ */
+int sf_attention_forward(const void* q, const void* k, const void* v, int64_t B, int64_t S, int64_t H, int64_t D,
+                         const float* cos, const float* sin, float scale, void* out, float* lse, void* q_rot,
+                         void* k_rot, void* stream);
+int sf_attention_backward(const void* q_rot, const void* k_rot, const void* v, const void* out, const void* grad_out,
+                          const float* lse, int64_t B, int64_t S, int64_t H, int64_t D, const float* cos,
+                          const float* sin, float scale, float* delta, void* dq, void* dk, void* dv, void* stream);
+
+/*
  * dst[b] = src[b]^T for `batch` row-major [rows, cols] matrices of 2- or
  * 4-byte elements (dst: [batch, cols, rows]): the contiguous transposed
  * operands of the attention products' derivatives (torch.bmm gets contiguous

@@ -451,8 +451,67 @@ def causal_attention(q, k, v, cos, sin) -> torch.Tensor:
     it.  The masked positions get -inf where the reference adds the dtype's lowest value: either way
     their probability is exactly 0."""
     if q.is_cuda:
+        if _fused_attention_takes(q, k, v, cos, sin):
+            return _FusedAttention.apply(q.contiguous(), k.contiguous(), v.contiguous(), cos.float().contiguous(),
+                                         sin.float().contiguous())
         return _causal_attention_device(q, k, v, cos, sin)
     return _causal_attention_torch(q, k, v, cos, sin)
+
+
+FUSED_MAX_S = 4096  # the longest row of the softmax passes that the double backward runs
+
+
+def _fused_attention_takes(q, k, v, cos, sin) -> bool:
+    """The calls sf_attention_* takes: bf16 q, k, v of one shape with heads of 64 or 128, within the sizes the
+    materialised path takes too (its passes run the double backward), 16-byte aligned."""
+    if q.dim() != 4 or q.shape != k.shape or q.shape != v.shape or q.numel() == 0:
+        return False
+    B, S, H, D = q.shape
+    return (D in (64, 128) and S <= FUSED_MAX_S and S * H * D * 2 < 2 ** 31 and B * S * H * (D // 8) < 2 ** 31
+            and all(t.is_cuda and t.device == q.device for t in (k, v, cos, sin))
+            and q.dtype == k.dtype == v.dtype == torch.bfloat16
+            and cos.numel() == S * D and sin.numel() == S * D
+            and all(not t.is_contiguous() or t.data_ptr() % 16 == 0 for t in (q, k, v, cos, sin)))
+
+
+class _FusedAttention(torch.autograd.Function):
+    """causal_attention of bf16 heads with the S x S products kept in registers (sf_attention_forward /
+    sf_attention_backward).  When the gradient itself is differentiated (create_graph, the Hutchinson probe)
+    the backward is that of the materialised path, whose passes are differentiable."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, cos, sin):
+        dev = L.require_device(q, k, v, cos, sin)
+        B, S, H, D = q.shape
+        out = torch.empty((B, S, H * D), dtype=q.dtype, device=dev)
+        lse = torch.empty((B * H, S), dtype=torch.float32, device=dev)
+        qr, kr = torch.empty_like(q), torch.empty_like(k)
+        with _prof.region("sf_attention_forward", 4 * q.numel() * q.element_size(), "B", dev):
+            L.check(L.lib().sf_attention_forward(L.ptr(q), L.ptr(k), L.ptr(v), B, S, H, D, L.ptr(cos), L.ptr(sin),
+                                                 D ** -0.5, L.ptr(out), L.ptr(lse), L.ptr(qr), L.ptr(kr),
+                                                 L.stream(dev)), "sf_attention_forward")
+        ctx.save_for_backward(q, k, v, cos, sin, qr, kr, out, lse)
+        return out
+
+    @staticmethod
+    def backward(ctx, go):
+        q, k, v, cos, sin, qr, kr, out, lse = ctx.saved_tensors
+        if torch.is_grad_enabled():  # create_graph
+            wanted = [t for t, n in zip((q, k, v), ctx.needs_input_grad) if n]
+            grads = iter(torch.autograd.grad(_causal_attention_device(q, k, v, cos, sin), wanted, go,
+                                             create_graph=True))
+            return (*(next(grads) if n else None for n in ctx.needs_input_grad[:3]), None, None)
+        dev = q.device
+        B, S, H, D = q.shape
+        go = _aligned(go.to(q.dtype))
+        delta = torch.empty_like(lse)
+        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+        with _prof.region("sf_attention_backward", 8 * q.numel() * q.element_size(), "B", dev):
+            L.check(L.lib().sf_attention_backward(L.ptr(qr), L.ptr(kr), L.ptr(v), L.ptr(out), L.ptr(go), L.ptr(lse),
+                                                  B, S, H, D, L.ptr(cos), L.ptr(sin), D ** -0.5, L.ptr(delta),
+                                                  L.ptr(dq), L.ptr(dk), L.ptr(dv), L.stream(dev)),
+                    "sf_attention_backward")
+        return dq, dk, dv, None, None
 
 
 def _causal_attention_torch(q, k, v, cos, sin) -> torch.Tensor:

@@ -1,0 +1,98 @@
+"""The fused bf16 causal attention (llama.causal_attention for heads of 64 or 128) against float64.
+
+Bar: the inputs are rotated in bf16 (both sides take the same rotated values), then p and ds round to bf16 once
+each before their product and the outputs round once: every output is a sum whose terms are off by at most 2^-8
+relative (2^-9 each for p or ds and for the stored result), so norm-wise 2^-8; 1e-2 leaves a factor of 2.5 for the
+rotation's own roundings in dq and dk."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _ref(q, k, v, cos, sin, go):
+    from sparseforge_amd import llama
+
+    B, S, H, D = q.shape
+    c, s = cos.to(q.dtype), sin.to(q.dtype)
+    rot = lambda t: llama._rotate(t.transpose(1, 2), c, s)  # noqa: E731
+    q, k, v = (t.detach().requires_grad_(True) for t in (q, k, v))
+    qd = rot(q).double()
+    kd = rot(k).double()
+    sc = qd @ kd.transpose(-1, -2) * D ** -0.5
+    sc = sc.masked_fill(torch.ones(S, S, dtype=torch.bool, device=q.device).triu(1), float("-inf"))
+    o = (sc.softmax(-1) @ v.transpose(1, 2).double()).transpose(1, 2).reshape(B, S, H * D)
+    return o, torch.autograd.grad(o, (q, k, v), go.double())
+
+
+@pytest.mark.parametrize("S", [1, 31, 64, 65, 128, 129, 200, 577, 1024])
+@pytest.mark.parametrize("B,H,D", [(2, 4, 64), (1, 3, 64), (1, 8, 128), (2, 1, 128)])
+def test_forward_and_gradients(cuda_device, S, B, H, D):
+    from sparseforge_amd import llama
+
+    g = torch.Generator(device=cuda_device).manual_seed(S + D)
+    q, k, v = (torch.randn(B, S, H, D, generator=g, device=cuda_device).to(torch.bfloat16).requires_grad_(True)
+               for _ in range(3))
+    go = torch.randn(B, S, H * D, generator=g, device=cuda_device).to(torch.bfloat16)
+    cos, sin = llama.rotary_tables(S, D, 10000.0, cuda_device)
+    assert llama._fused_attention_takes(q, k, v, cos, sin)
+    o = llama.causal_attention(q, k, v, cos, sin)
+    grads = torch.autograd.grad(o, (q, k, v), go)
+    ro, rg = _ref(q, k, v, cos, sin, go)
+    for got, want in zip((o, *grads), (ro, *rg)):
+        got, want = got.detach(), want.detach()
+        assert torch.isfinite(got).all()
+        err = float((got.double() - want.double()).norm() / want.double().norm().clamp_min(1e-30))
+        assert err < 1e-2 or float(want.double().norm()) < 1e-3, err
+
+
+def test_large_scores_and_nan(cuda_device):
+    """Rows whose scores are far apart (one key takes all), and a NaN that stays in its head's later rows."""
+    from sparseforge_amd import llama
+
+    S, D = 150, 64
+    q, k, v = (torch.randn(1, S, 2, D, device=cuda_device) for _ in range(3))
+    q, k, v = (t.to(torch.bfloat16) for t in (q * 60, k * 60, v))
+    go = torch.randn(1, S, 2 * D, device=cuda_device).to(torch.bfloat16)
+    cos, sin = llama.rotary_tables(S, D, 10000.0, cuda_device)
+    o = llama.causal_attention(q, k, v, cos, sin)
+    ro, _ = _ref(q, k, v, cos, sin, go)
+    assert torch.isfinite(o).all()
+    assert float((o.double() - ro).norm() / ro.norm()) < 1e-2
+    v2 = v.clone()
+    v2[0, 100, 1, 3] = float("nan")
+    o2 = llama.causal_attention(q, k, v2, cos, sin).view(S, 2, D)
+    assert torch.isfinite(o2[:, 0]).all() and torch.isfinite(o2[:64, 1]).all() and torch.isnan(o2[100:, 1, 3]).all()
+
+
+def test_double_backward_takes_the_materialised_path(cuda_device):
+    """With create_graph the gradients equal the materialised path's, and so do the second derivatives."""
+    from sparseforge_amd import llama
+
+    B, S, H, D = 1, 96, 2, 64
+    g = torch.Generator(device=cuda_device).manual_seed(3)
+    base = [torch.randn(B, S, H, D, generator=g, device=cuda_device).to(torch.bfloat16) for _ in range(3)]
+    probes = [torch.randn(B, S, H, D, generator=g, device=cuda_device) for _ in range(3)]
+    w = torch.randn(B, S, H * D, generator=g, device=cuda_device)
+    cos, sin = llama.rotary_tables(S, D, 10000.0, cuda_device)
+    outs = []
+    for fn in (llama.causal_attention, llama._causal_attention_device):
+        x = [t.clone().requires_grad_(True) for t in base]
+        loss = (fn(*x, cos, sin).float() * w).sum()  # linear in the output: the same upstream gradient
+        grads = torch.autograd.grad(loss, x, create_graph=True)
+        dot = sum((a.float() * p).sum() for a, p in zip(grads, probes))
+        outs.append((*grads, *torch.autograd.grad(dot, x)))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+
+
+def test_calls_outside_the_fused_path(cuda_device):
+    """float32, another head size and unaligned operands run the materialised path as before."""
+    from sparseforge_amd import llama
+
+    for D, dt in ((64, torch.float32), (32, torch.bfloat16), (96, torch.bfloat16)):
+        q, k, v = (torch.randn(1, 40, 2, D, device=cuda_device).to(dt) for _ in range(3))
+        cos, sin = llama.rotary_tables(40, D, 10000.0, cuda_device)
+        assert not llama._fused_attention_takes(q, k, v, cos, sin)
+        assert torch.equal(llama.causal_attention(q, k, v, cos, sin),
+                           llama._causal_attention_device(q, k, v, cos, sin))
