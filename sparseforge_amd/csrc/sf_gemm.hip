@@ -48,48 +48,7 @@ constexpr int kWaveM = 128;
 constexpr int kWaveN = 128;
 constexpr int kFragM = kWaveM / 32;  // 4
 constexpr int kFragN = kWaveN / 32;  // 4
-constexpr int kGroupM = 8;           // M-tiles per L2 band
-constexpr int kXcds = 8;
 constexpr int kEpiPitch = 132;     // f32 row pitch of the epilogue staging (64 rows x 128 cols per wave)
-
-struct GemmArgs {
-  int64_t M, N, K1, K2;
-  const void* A1;
-  int64_t lda1;
-  const void* A2;
-  int64_t lda2;
-  const void* B1;
-  int64_t ldb1;
-  const void* B2;
-  int64_t ldb2;
-  const void* bmask;  // effective mask of B1 (element dtype, B1's layout and ld)
-  float bscale;       // 1: none
-  int has_scale;
-  void* C;
-  int64_t ldc;
-  int c_dtype;
-  const void* bias;  // [N], element dtype or f32
-  int bias_dtype;
-  const void* emask;  // [M, N] row-major with ld = ldc: C *= emask
-  const void* dw;     // [M, N]: C += decay * dw * (emask < 0.5)
-  float decay;
-  int accumulate;  // C += result
-  int c_aligned;   // C is 16-byte aligned
-  int64_t tiles_m, tiles_n;
-  int splits;            // K splits (1: the kernel writes C itself)
-  int64_t split_stages;  // segment-1 stages per split
-  float* partial;        // splits > 1: [splits][M][N] f32 partial sums
-  // block-sparse-16 B1 (B layouts 2 / 3): B1 is the blocks array, b_map its block map
-  const int32_t* b_map;
-  int64_t b_map_rows, b_map_cols;
-  // block-sparse-16 C: the epilogue writes only the blocks c_map lists, into c_blocks
-  void* c_blocks;
-  const int32_t* c_map;
-  int64_t c_map_rows, c_map_cols;
-  int64_t ldbm;      // leading dimension of a K-major byte mask ([N][K1])
-  int bmask_kmajor;  // bmask is K-major (input gradient: B = W^T, mask given transposed)
-  int dma_mask_ok;   // the byte mask can be copied 16 bytes at a time (bf16 direct kernel)
-};
 
 // Element traits.  bf16 uses v_mfma_f32_32x32x16_bf16 (8 k-values per lane),
 // f32 uses v_mfma_f32_32x32x2_f32 (1 k-value per lane).
@@ -496,18 +455,6 @@ struct BsrLoader {
     }
   }
 };
-
-// Tile coordinates of workgroup `pid` (XCD-contiguous ranges, bands of kGroupM M-tiles).
-__device__ __forceinline__ void tile_coords(int64_t pid, int64_t tiles_m, int64_t tiles_n, int64_t& tm, int64_t& tn) {
-  const int64_t total = tiles_m * tiles_n;
-  if (total % kXcds == 0) pid = (pid % kXcds) * (total / kXcds) + pid / kXcds;
-  const int64_t band = kGroupM * tiles_n;
-  const int64_t first_m = (pid / band) * kGroupM;
-  const int64_t gm = tiles_m - first_m < kGroupM ? tiles_m - first_m : kGroupM;
-  const int64_t r = pid % band;
-  tm = first_m + r % gm;
-  tn = r / gm;
-}
 
 // Epilogue shared by the GEMM kernels: the 4 x 4 accumulator blocks of each
 // wave (its 128 x 128 share of the 256 x 256 tile) go to C, a split-K partial
@@ -1426,44 +1373,6 @@ __global__ void __launch_bounds__(kThreads, 1) gemm_bf16_kernel(GemmArgs g) {
   gemm_epilogue<T>(g, acc, smem, m0, n0, kz);
 }
 
-// Split-K reduction: C = epilogue(sum over splits of the f32 partials), the
-// splits summed in index order (deterministic), then the same output
-// rounding, bias, mask product / decay term and accumulation as the GEMM
-// epilogue.
-__global__ void __launch_bounds__(256) splitk_reduce_kernel(GemmArgs g, int elem_dtype) {
-  const int64_t total = g.M * g.N;
-  const bool cbf = g.c_dtype == SF_DTYPE_BF16;
-  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t row = idx / g.N, col = idx - row * g.N;
-    float x = 0.0f;
-    for (int z = 0; z < g.splits; ++z) x += g.partial[z * total + idx];
-    const int64_t o = row * g.ldc + col;
-    if (cbf) x = hround(x);
-    if (g.bias) {
-      const float b = load_elem(g.bias, col, g.bias_dtype);
-      x = cbf ? hround(x + b) : x + b;
-    }
-    if (g.emask) {
-      const float em = load_elem(g.emask, o, elem_dtype);
-      if (g.dw) {
-        if (em < 0.5f) {
-          float d = g.decay * load_elem(g.dw, o, elem_dtype);
-          if (cbf) d = hround(d);
-          x = cbf ? hround(x + d) : x + d;
-        }
-      } else {
-        x = cbf ? hround(x * em) : x * em;
-      }
-    }
-    if (g.accumulate) x = load_elem(g.C, o, g.c_dtype) + x;
-    if (cbf)
-      static_cast<uint16_t*>(g.C)[o] = hbits(x);
-    else
-      static_cast<float*>(g.C)[o] = x;
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Block-sparse-16 products on bf16 operands (the BSR layout of
 // convert_to_block_sparse plus its block map), DMA-staged like gemm_bf16_kernel.
@@ -1689,9 +1598,7 @@ int launch_gemm(const GemmArgs& g, hipStream_t st) {
   hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(tiles * g.splits)), dim3(kThreads), smem, st, g);
   if (int rc = launch_status("sf_gemm")) return rc;
   if (g.splits > 1) {
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3(static_cast<unsigned>(elementwise_grid(g.M * g.N, 256))),
-                       dim3(256), 0, st, g, Tr<T>::DT);
-    return launch_status("sf_gemm (split-K reduce)");
+    return launch_splitk_reduce(g, Tr<T>::DT, st, "sf_gemm (split-K reduce)");
   }
   return SF_OK;
 }
@@ -2212,9 +2119,7 @@ int launch_skinny(const sf_gemm_desc* d, GemmArgs g, hipStream_t st) {
   if (int rc = launch_status("sf_gemm (skinny)")) return rc;
   g.splits = sp;
   g.partial = a.partial;
-  hipLaunchKernelGGL(splitk_reduce_kernel, dim3(static_cast<unsigned>(elementwise_grid(g.M * g.N, 256))), dim3(256), 0,
-                     st, g, SF_DTYPE_BF16);
-  return launch_status("sf_gemm (skinny reduce)");
+  return launch_splitk_reduce(g, SF_DTYPE_BF16, st, "sf_gemm (skinny reduce)");
 }
 
 template <typename T, int MASK>
@@ -2239,6 +2144,11 @@ int dispatch_layouts(const sf_gemm_desc* d, const GemmArgs& g, hipStream_t st) {
 
 bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// A product the f32 kernels of sf_gemm_f32.hip take.
+bool f32_dense(const sf_gemm_desc* d) {
+  return d->dtype == SF_DTYPE_F32 && d->b_format == SF_BFMT_DENSE && !d->bmask && !d->c_blocks;
+}
+
 // K splits for a GEMM whose tile grid would leave most of the 256 CUs idle:
 // enough splits to give about one workgroup per CU, each split keeping at
 // least 8 stages of K, at most 16 splits.
@@ -2262,6 +2172,7 @@ extern "C" size_t sf_gemm_workspace_size(const sf_gemm_desc* d) {
   if (!d || d->M <= 0 || d->N <= 0 || d->K1 <= 0) return 0;
   if (d->dtype != SF_DTYPE_BF16 && d->dtype != SF_DTYPE_F32) return 0;
   if (skinny_ok(d)) return skinny_workspace(d);
+  if (f32_dense(d)) return gemm_f32_workspace(d->M, d->N, d->K1);
   const int sp = choose_splits(d);
   return sp > 1 ? static_cast<size_t>(sp) * d->M * d->N * sizeof(float) : 0;
 }
@@ -2397,6 +2308,7 @@ extern "C" int sf_gemm(const sf_gemm_desc* d, void* stream) {
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (skinny_ok(d) && d->workspace && d->workspace_bytes >= skinny_workspace(d) && al16(d->workspace))
     return launch_skinny(d, g, st);
+  if (f32_dense(d)) return launch_gemm_f32(g, d->a_layout, d->b_layout, d->workspace, d->workspace_bytes, st);
   const bool bf = d->dtype == SF_DTYPE_BF16;
   if (g.bmask && d->bmask_bytes)
     return bf ? dispatch_layouts<uint16_t, kMaskByte>(d, g, st) : dispatch_layouts<float, kMaskByte>(d, g, st);

@@ -66,7 +66,69 @@ __device__ __forceinline__ V4 bload(Rsrc r, uint32_t voff, uint32_t soff) {
 
 __device__ __forceinline__ float load_elem(const void* p, int64_t i, int dtype) { return load_as_f32(p, i, dtype); }
 
+constexpr int kGroupM = 8;  // M-tiles per L2 band
+constexpr int kXcds = 8;
+
+// Tile coordinates of workgroup `pid` (XCD-contiguous ranges, bands of kGroupM M-tiles).
+__device__ __forceinline__ void tile_coords(int64_t pid, int64_t tiles_m, int64_t tiles_n, int64_t& tm, int64_t& tn) {
+  const int64_t total = tiles_m * tiles_n;
+  if (total % kXcds == 0) pid = (pid % kXcds) * (total / kXcds) + pid / kXcds;
+  const int64_t band = kGroupM * tiles_n;
+  const int64_t first_m = (pid / band) * kGroupM;
+  const int64_t gm = tiles_m - first_m < kGroupM ? tiles_m - first_m : kGroupM;
+  const int64_t r = pid % band;
+  tm = first_m + r % gm;
+  tn = r / gm;
+}
+
 }  // namespace
+
+// A product of sf_gemm as its kernels take it.
+struct GemmArgs {
+  int64_t M, N, K1, K2;
+  const void* A1;
+  int64_t lda1;
+  const void* A2;
+  int64_t lda2;
+  const void* B1;
+  int64_t ldb1;
+  const void* B2;
+  int64_t ldb2;
+  const void* bmask;  // effective mask of B1 (element dtype, B1's layout and ld)
+  float bscale;       // 1: none
+  int has_scale;
+  void* C;
+  int64_t ldc;
+  int c_dtype;
+  const void* bias;  // [N], element dtype or f32
+  int bias_dtype;
+  const void* emask;  // [M, N] row-major with ld = ldc: C *= emask
+  const void* dw;     // [M, N]: C += decay * dw * (emask < 0.5)
+  float decay;
+  int accumulate;  // C += result
+  int c_aligned;   // C is 16-byte aligned
+  int64_t tiles_m, tiles_n;
+  int splits;            // K splits (1: the kernel writes C itself)
+  int64_t split_stages;  // segment-1 stages per split
+  float* partial;        // splits > 1: [splits][M][N] f32 partial sums
+  // block-sparse-16 B1 (B layouts 2 / 3): B1 is the blocks array, b_map its block map
+  const int32_t* b_map;
+  int64_t b_map_rows, b_map_cols;
+  // block-sparse-16 C: the epilogue writes only the blocks c_map lists, into c_blocks
+  void* c_blocks;
+  const int32_t* c_map;
+  int64_t c_map_rows, c_map_cols;
+  int64_t ldbm;      // leading dimension of a K-major byte mask ([N][K1])
+  int bmask_kmajor;  // bmask is K-major (input gradient: B = W^T, mask given transposed)
+  int dma_mask_ok;   // the byte mask can be copied 16 bytes at a time (bf16 direct kernel)
+};
+
+// C = epilogue(sum of the K splits' partials) (sf_splitk.hip).
+int launch_splitk_reduce(const GemmArgs& g, int elem_dtype, hipStream_t st, const char* what);
+
+// The f32 product of dense, unmasked operands (sf_gemm_f32.hip): its workspace for K-split partials, and the launch.
+size_t gemm_f32_workspace(int64_t M, int64_t N, int64_t K);
+int launch_gemm_f32(GemmArgs g, int a_layout, int b_layout, void* workspace, size_t workspace_bytes, hipStream_t st);
 
 // y [N tokens, M out] = x W^T (+ A2/B2 low-rank term, + bias), W packed 2:4.
 struct Gemm24Args {

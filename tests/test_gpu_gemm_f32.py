@@ -1,0 +1,52 @@
+"""The f32 products (sf_gemm on dense f32 operands) at the edges of their tiles and K splits, all three layouts, with
+the second K segment and every epilogue, against float64 (conftest.gemm_err: 1e-5 of the output scale; a float32 sum
+of K terms is off by about sqrt(K) 2^-24 of the terms' scale, K at most 8168 here)."""
+import pytest
+import torch
+
+from conftest import gemm_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _mk(g, dev, *shape):
+    return torch.randn(*shape, generator=g, device=dev)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (4, 4, 4), (32, 32, 36), (33, 16, 768), (16, 768, 8168), (3072, 16, 1000), (100, 132, 68),
+    (129, 65, 260), (1021, 768, 3072), (768, 3072, 1021), (260, 2052, 33 * 4), (8168, 20, 768),
+])
+@pytest.mark.parametrize("layout", ["nt", "nn", "tn"])
+def test_layouts(cuda_device, M, N, K, layout):
+    from sparseforge_amd import linear as lin
+
+    if layout == "nt" and K % 4 or layout != "nt" and N % 4 or layout == "tn" and M % 4 or layout == "nn" and K % 4:
+        pytest.skip("rows of whole 16-byte vectors only")
+    g = torch.Generator(device=cuda_device).manual_seed(M + N + K)
+    A = _mk(g, cuda_device, *((K, M) if layout == "tn" else (M, K)))
+    B = _mk(g, cuda_device, *((N, K) if layout == "nt" else (K, N)))
+    got = getattr(lin, "mm_" + layout)(A, B)
+    a = A.double().t() if layout == "tn" else A.double()
+    b = B.double().t() if layout == "nt" else B.double()
+    assert gemm_err(got, a @ b, torch.float32) <= 1.0
+
+
+@pytest.mark.parametrize("M,N,K,R", [(64, 96, 128, 4), (1000, 260, 516, 20), (48, 32, 8192, 64)])
+def test_segment_bias_mask_accumulate(cuda_device, M, N, K, R):
+    from sparseforge_amd import linear as lin
+
+    g = torch.Generator(device=cuda_device).manual_seed(M)
+    A, B = _mk(g, cuda_device, M, K), _mk(g, cuda_device, N, K)
+    z, S, bias = _mk(g, cuda_device, M, R), _mk(g, cuda_device, N, R), _mk(g, cuda_device, N)
+    E, C, W = torch.rand(M, N, generator=g, device=cuda_device), _mk(g, cuda_device, M, N), _mk(g, cuda_device, M, N)
+    prod = A.double() @ B.double().t() + z.double() @ S.double().t()
+    kw = {"A2": z, "B2": S, "K2": R}
+    assert gemm_err(lin.mm_nt(A, B, bias=bias, **kw), prod + bias.double(), torch.float32) <= 1.0
+    assert gemm_err(lin.mm_nt(A, B, emask=E, **kw), prod * E.double(), torch.float32) <= 1.0
+    got = lin.mm_nt(A, B, emask=E, dw=W, decay=0.25, **kw)
+    assert gemm_err(got, prod + 0.25 * W.double() * (E < 0.5), torch.float32) <= 1.0
+    got = lin.mm_nt(A, B, out=C.clone(), accumulate=True, **kw)
+    assert gemm_err(got, prod + C.double(), torch.float32) <= 1.0
+    for cap in (1, 2):  # fewer splits than planned: the workspace a caller gives
+        assert gemm_err(lin.mm_nt(A, B, max_splits=cap, **kw), prod, torch.float32) <= 1.0
