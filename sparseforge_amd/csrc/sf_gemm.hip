@@ -472,7 +472,6 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, const f32x16_t 
   // (bias, mask product, decay term, accumulation) are read coalesced.
   float* ep = reinterpret_cast<float*>(smem) + wave * (64 * kEpiPitch);
   const int64_t wrow0 = m0 + wm * kWaveM, wcol0 = n0 + wn * kWaveN;
-  const bool cbf = g.c_dtype == SF_DTYPE_BF16;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     __syncthreads();
@@ -496,103 +495,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, const f32x16_t 
       const float4 p1 = *reinterpret_cast<const float4*>(ep + r * kEpiPitch + c + 4);
       v[0] = p0.x; v[1] = p0.y; v[2] = p0.z; v[3] = p0.w;
       v[4] = p1.x; v[5] = p1.y; v[6] = p1.z; v[7] = p1.w;
-      if (g.c_blocks) {
-        // block-sparse C (the SDDMM weight gradient): only kept 16 x 16 blocks are written,
-        // row (row % 16) of block c_map[row / 16][col / 16], 8 columns at a time
-        const int64_t bi = (row / 16 < g.c_map_rows && col / 16 < g.c_map_cols)
-                               ? g.c_map[(row / 16) * g.c_map_cols + col / 16] : -1;
-        if (bi >= 0) {
-          const int64_t o = bi * 256 + (row % 16) * 16 + (col % 16);
-          if (g.c_dtype == SF_DTYPE_BF16) {
-            *reinterpret_cast<uint4*>(static_cast<uint16_t*>(g.c_blocks) + o) =
-                make_uint4(pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7]));
-          } else {
-            float* cp = static_cast<float*>(g.c_blocks) + o;
-            *reinterpret_cast<float4*>(cp) = make_float4(v[0], v[1], v[2], v[3]);
-            *reinterpret_cast<float4*>(cp + 4) = make_float4(v[4], v[5], v[6], v[7]);
-          }
-        }
-        continue;
-      }
-      if (g.splits > 1) {
-        // split-K: raw f32 partial sums; sf_gemm's reduce kernel applies the epilogue
-        float* pp = g.partial + (kz * g.M + row) * g.N + col;
-        if (col + 8 <= g.N && (g.N & 3) == 0) {
-          *reinterpret_cast<float4*>(pp) = make_float4(v[0], v[1], v[2], v[3]);
-          *reinterpret_cast<float4*>(pp + 4) = make_float4(v[4], v[5], v[6], v[7]);
-        } else {
-          for (int q = 0; q < 8 && col + q < g.N; ++q) pp[q] = v[q];
-        }
-        continue;
-      }
-      const int64_t off = row * g.ldc + col;
-      const bool vec = g.c_aligned && col + 8 <= g.N && (off & 7) == 0;
-      if (!g.emask && vec) {
-        // result of the matmul in the output dtype, then + bias (rounded again), then + C when
-        // accumulating: the per-element sequence below, 8 outputs at a time
-        if (g.bias) {
-#pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            const float b = load_elem(g.bias, col + q, g.bias_dtype);
-            v[q] = cbf ? hround(v[q]) + b : v[q] + b;
-          }
-        }
-        if (g.accumulate) {
-          float c[8];
-          if (cbf) {
-            const uint4 cw = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(g.C) + off);
-            const uint32_t w4[4] = {cw.x, cw.y, cw.z, cw.w};
-#pragma unroll
-            for (int q = 0; q < 8; ++q) c[q] = bf16_to_f32(static_cast<uint16_t>(w4[q >> 1] >> (16 * (q & 1))));
-          } else {
-            const float4 c0 = *reinterpret_cast<const float4*>(static_cast<const float*>(g.C) + off);
-            const float4 c1 = *reinterpret_cast<const float4*>(static_cast<const float*>(g.C) + off + 4);
-            c[0] = c0.x; c[1] = c0.y; c[2] = c0.z; c[3] = c0.w;
-            c[4] = c1.x; c[5] = c1.y; c[6] = c1.z; c[7] = c1.w;
-          }
-#pragma unroll
-          for (int q = 0; q < 8; ++q) {
-            const float x = cbf ? hround(v[q]) : v[q];  // the product (+ bias) in the output dtype
-            v[q] = c[q] + x;
-          }
-        }
-        if (cbf) {
-          *reinterpret_cast<uint4*>(static_cast<uint16_t*>(g.C) + off) =
-              make_uint4(pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7]));
-        } else {
-          float* cp = static_cast<float*>(g.C) + off;
-          *reinterpret_cast<float4*>(cp) = make_float4(v[0], v[1], v[2], v[3]);
-          *reinterpret_cast<float4*>(cp + 4) = make_float4(v[4], v[5], v[6], v[7]);
-        }
-        continue;
-      }
-      const int edt = Tr<T>::DT;
-      for (int q = 0; q < 8; ++q) {
-        if (col + q >= g.N) break;
-        const int64_t o = off + q;
-        float x = cbf ? hround(v[q]) : v[q];
-        if (g.bias) {
-          const float b = load_elem(g.bias, col + q, g.bias_dtype);
-          x = cbf ? hround(x + b) : x + b;
-        }
-        if (g.emask) {
-          const float em = load_elem(g.emask, o, edt);
-          if (g.dw) {
-            if (em < 0.5f) {
-              float d = g.decay * load_elem(g.dw, o, edt);
-              if (cbf) d = hround(d);
-              x = cbf ? hround(x + d) : x + d;
-            }
-          } else {
-            x = cbf ? hround(x * em) : x * em;
-          }
-        }
-        if (g.accumulate) x = load_elem(g.C, o, g.c_dtype) + x;
-        if (cbf)
-          static_cast<uint16_t*>(g.C)[o] = hbits(x);
-        else
-          static_cast<float*>(g.C)[o] = x;
-      }
+      store_c8<Tr<T>::DT>(g, row, col, kz, v);
     }
   }
 }
@@ -2149,6 +2052,12 @@ bool f32_dense(const sf_gemm_desc* d) {
   return d->dtype == SF_DTYPE_F32 && d->b_format == SF_BFMT_DENSE && !d->bmask && !d->c_blocks;
 }
 
+// A product the 128 x 128 tiles of sf_gemm_mid.hip take.
+bool mid_dense(const sf_gemm_desc* d) {
+  return d->dtype == SF_DTYPE_BF16 && d->b_format == SF_BFMT_DENSE && !d->bmask && d->K1 > 0;
+}
+constexpr int kMidMaxSplits = 16;
+
 // K splits for a GEMM whose tile grid would leave most of the 256 CUs idle:
 // enough splits to give about one workgroup per CU, each split keeping at
 // least 8 stages of K, at most 16 splits.
@@ -2173,7 +2082,9 @@ extern "C" size_t sf_gemm_workspace_size(const sf_gemm_desc* d) {
   if (d->dtype != SF_DTYPE_BF16 && d->dtype != SF_DTYPE_F32) return 0;
   if (skinny_ok(d)) return skinny_workspace(d);
   if (f32_dense(d)) return gemm_f32_workspace(d->M, d->N, d->K1);
-  const int sp = choose_splits(d);
+  const int big = choose_splits(d);
+  int sp = mid_dense(d) ? gemm_mid_splits(d->M, d->N, d->K1, d->c_blocks ? 1 : kMidMaxSplits, big) : 0;
+  if (sp == 0) sp = big;
   return sp > 1 ? static_cast<size_t>(sp) * d->M * d->N * sizeof(float) : 0;
 }
 
@@ -2309,6 +2220,14 @@ extern "C" int sf_gemm(const sf_gemm_desc* d, void* stream) {
   if (skinny_ok(d) && d->workspace && d->workspace_bytes >= skinny_workspace(d) && al16(d->workspace))
     return launch_skinny(d, g, st);
   if (f32_dense(d)) return launch_gemm_f32(g, d->a_layout, d->b_layout, d->workspace, d->workspace_bytes, st);
+  if (mid_dense(d)) {
+    // as many K splits as the workspace holds partials for
+    const size_t per = static_cast<size_t>(d->M) * d->N * sizeof(float);
+    const size_t cap = d->workspace && al16(d->workspace) && !d->c_blocks ? d->workspace_bytes / per : 1;
+    const int sp = gemm_mid_splits(d->M, d->N, d->K1, cap > kMidMaxSplits ? kMidMaxSplits : (cap < 1 ? 1 : (int)cap),
+                                   g.splits);
+    if (sp > 0) return launch_gemm_mid(g, d->a_layout, d->b_layout, sp, d->workspace, st);
+  }
   const bool bf = d->dtype == SF_DTYPE_BF16;
   if (g.bmask && d->bmask_bytes)
     return bf ? dispatch_layouts<uint16_t, kMaskByte>(d, g, st) : dispatch_layouts<float, kMaskByte>(d, g, st);

@@ -123,8 +123,136 @@ struct GemmArgs {
   int dma_mask_ok;   // the byte mask can be copied 16 bytes at a time (bf16 direct kernel)
 };
 
+namespace {
+// 8 consecutive columns of one row of a product (its f32 sums v): to the K split's partials, to the kept blocks of a
+// block-sparse C, or through the epilogue (output rounding, bias, mask product / decay term, accumulation) to C.
+// EDT: dtype of emask and dw.
+template <int EDT>
+__device__ __forceinline__ void store_c8(const GemmArgs& g, int64_t row, int64_t col, int64_t kz, float (&v)[8]) {
+  const bool cbf = g.c_dtype == SF_DTYPE_BF16;
+  if (g.c_blocks) {
+    // block-sparse C (the SDDMM weight gradient): only kept 16 x 16 blocks are written,
+    // row (row % 16) of block c_map[row / 16][col / 16], 8 columns at a time
+    const int64_t bi = (row / 16 < g.c_map_rows && col / 16 < g.c_map_cols)
+                           ? g.c_map[(row / 16) * g.c_map_cols + col / 16] : -1;
+    if (bi >= 0) {
+      const int64_t o = bi * 256 + (row % 16) * 16 + (col % 16);
+      if (g.c_dtype == SF_DTYPE_BF16) {
+        *reinterpret_cast<uint4*>(static_cast<uint16_t*>(g.c_blocks) + o) =
+            make_uint4(pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7]));
+      } else {
+        float* cp = static_cast<float*>(g.c_blocks) + o;
+        *reinterpret_cast<float4*>(cp) = make_float4(v[0], v[1], v[2], v[3]);
+        *reinterpret_cast<float4*>(cp + 4) = make_float4(v[4], v[5], v[6], v[7]);
+      }
+    }
+    return;
+  }
+  if (g.splits > 1) {
+    // split-K: raw f32 partial sums; sf_gemm's reduce kernel applies the epilogue
+    float* pp = g.partial + (kz * g.M + row) * g.N + col;
+    if (col + 8 <= g.N && (g.N & 3) == 0) {
+      *reinterpret_cast<float4*>(pp) = make_float4(v[0], v[1], v[2], v[3]);
+      *reinterpret_cast<float4*>(pp + 4) = make_float4(v[4], v[5], v[6], v[7]);
+    } else {
+      for (int q = 0; q < 8 && col + q < g.N; ++q) pp[q] = v[q];
+    }
+    return;
+  }
+  const int64_t off = row * g.ldc + col;
+  const bool vec = g.c_aligned && col + 8 <= g.N && (off & 7) == 0 &&
+                   (!g.emask || (reinterpret_cast<uintptr_t>(g.emask) & 15u) == 0);
+  if (!g.dw && vec) {
+    // result of the matmul in the output dtype, then + bias (rounded again), then + C when
+    // accumulating: the per-element sequence below, 8 outputs at a time
+    if (g.bias) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const float b = load_elem(g.bias, col + q, g.bias_dtype);
+        v[q] = cbf ? hround(v[q]) + b : v[q] + b;
+      }
+    }
+    if (g.emask) {  // times the effective mask, after the product (+ bias) is rounded
+      float em[8];
+      if constexpr (EDT == SF_DTYPE_BF16) {
+        const uint4 ew = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(g.emask) + off);
+        const uint32_t w4[4] = {ew.x, ew.y, ew.z, ew.w};
+#pragma unroll
+        for (int q = 0; q < 8; ++q) em[q] = (q & 1) ? hi_f(w4[q >> 1]) : lo_f(w4[q >> 1]);
+      } else {
+        const float4 e0 = *reinterpret_cast<const float4*>(static_cast<const float*>(g.emask) + off);
+        const float4 e1 = *reinterpret_cast<const float4*>(static_cast<const float*>(g.emask) + off + 4);
+        em[0] = e0.x; em[1] = e0.y; em[2] = e0.z; em[3] = e0.w; em[4] = e1.x; em[5] = e1.y; em[6] = e1.z; em[7] = e1.w;
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] = (cbf ? hround(v[q]) : v[q]) * em[q];
+    }
+    if (g.accumulate) {
+      float c[8];
+      if (cbf) {
+        const uint4 cw = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(g.C) + off);
+        const uint32_t w4[4] = {cw.x, cw.y, cw.z, cw.w};
+#pragma unroll
+        for (int q = 0; q < 8; ++q) c[q] = bf16_to_f32(static_cast<uint16_t>(w4[q >> 1] >> (16 * (q & 1))));
+      } else {
+        const float4 c0 = *reinterpret_cast<const float4*>(static_cast<const float*>(g.C) + off);
+        const float4 c1 = *reinterpret_cast<const float4*>(static_cast<const float*>(g.C) + off + 4);
+        c[0] = c0.x; c[1] = c0.y; c[2] = c0.z; c[3] = c0.w;
+        c[4] = c1.x; c[5] = c1.y; c[6] = c1.z; c[7] = c1.w;
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const float x = cbf ? hround(v[q]) : v[q];  // the product (+ bias) in the output dtype
+        v[q] = c[q] + x;
+      }
+    }
+    if (cbf) {
+      *reinterpret_cast<uint4*>(static_cast<uint16_t*>(g.C) + off) =
+          make_uint4(pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7]));
+    } else {
+      float* cp = static_cast<float*>(g.C) + off;
+      *reinterpret_cast<float4*>(cp) = make_float4(v[0], v[1], v[2], v[3]);
+      *reinterpret_cast<float4*>(cp + 4) = make_float4(v[4], v[5], v[6], v[7]);
+    }
+    return;
+  }
+  const int edt = EDT;
+  for (int q = 0; q < 8; ++q) {
+    if (col + q >= g.N) break;
+    const int64_t o = off + q;
+    float x = cbf ? hround(v[q]) : v[q];
+    if (g.bias) {
+      const float b = load_elem(g.bias, col + q, g.bias_dtype);
+      x = cbf ? hround(x + b) : x + b;
+    }
+    if (g.emask) {
+      const float em = load_elem(g.emask, o, edt);
+      if (g.dw) {
+        if (em < 0.5f) {
+          float d = g.decay * load_elem(g.dw, o, edt);
+          if (cbf) d = hround(d);
+          x = cbf ? hround(x + d) : x + d;
+        }
+      } else {
+        x = cbf ? hround(x * em) : x * em;
+      }
+    }
+    if (g.accumulate) x = load_elem(g.C, o, g.c_dtype) + x;
+    if (cbf)
+      static_cast<uint16_t*>(g.C)[o] = hbits(x);
+    else
+      static_cast<float*>(g.C)[o] = x;
+  }
+}
+}  // namespace
+
 // C = epilogue(sum of the K splits' partials) (sf_splitk.hip).
 int launch_splitk_reduce(const GemmArgs& g, int elem_dtype, hipStream_t st, const char* what);
+
+// The bf16 product of dense, unmasked operands on 128 x 128 tiles (sf_gemm_mid.hip): K splits it would take (0: the
+// 256 x 256 tiles are the better choice), and its launch.
+int gemm_mid_splits(int64_t M, int64_t N, int64_t K, int max_splits, int big_splits);
+int launch_gemm_mid(GemmArgs g, int a_layout, int b_layout, int splits, void* workspace, hipStream_t st);
 
 // The f32 product of dense, unmasked operands (sf_gemm_f32.hip): its workspace for K-split partials, and the launch.
 size_t gemm_f32_workspace(int64_t M, int64_t N, int64_t K);
