@@ -19,6 +19,7 @@ import torch
 
 from . import _lib as L
 from . import profiling as _prof
+from .linear import apply_in_backward
 
 
 class _KL(torch.autograd.Function):
@@ -44,7 +45,7 @@ class _KL(torch.autograd.Function):
         s2, t2, lse, scale = ctx.saved_tensors
         # a Function of its own, so that torch.autograd.grad(..., create_graph=True) (the Hutchinson
         # Hessian-vector product) differentiates the KL gradient as the reference's torch ops are
-        gs = _KLGrad.apply(s2, t2, lse, scale, g, ctx.temperature)
+        gs = apply_in_backward(_KLGrad, s2, t2, lse, scale, g, ctx.temperature)
         return gs, None, None, None
 
 

@@ -263,7 +263,7 @@ def update_mask_multi(p: L.MaskParams, q: float, jobs: list[MaskJob], stages: in
     dev = jobs[0].ops.device()
     first = jobs[0].ops
     dts = [first.dt(t) for t in (first.weight, first.hessian, first.aux, first.mask, first.frozen)]
-    nbytes = 0
+    nbytes, timed = 0, _prof.active()
     for j in jobs:
         o = j.ops
         if o.device() != dev:
@@ -277,6 +277,8 @@ def update_mask_multi(p: L.MaskParams, q: float, jobs: list[MaskJob], stages: in
             raise TypeError("sample indices must be a 1-D int64 tensor")
         # algorithmic bytes: the statistics read the score operands, the update reads them again and
         # reads + writes the mask (and the frozen flags when freezing)
+        if not timed:
+            continue
         if stages & L.MULTI_STATS:
             nbytes += o.score_bytes()
         if stages & L.MULTI_UPDATE:
@@ -510,25 +512,31 @@ class LayerPipeline:
     """
 
     def __init__(self, device: torch.device, n: int = 4):
-        key = (device.index, n)
+        self.device, self.n = device, n
+        self.streams = None  # forked on first use: most updates batch every layer and need no side stream
+        self.i = 0
+
+    def _fork(self) -> None:
+        key = (self.device.index, self.n)
         if key not in _SIDE_STREAMS:
-            _SIDE_STREAMS[key] = [torch.cuda.Stream(device=device) for _ in range(n)]
-        self.main = torch.cuda.current_stream(device)
+            _SIDE_STREAMS[key] = [torch.cuda.Stream(device=self.device) for _ in range(self.n)]
+        self.main = torch.cuda.current_stream(self.device)
         self.streams = _SIDE_STREAMS[key]
         start = torch.cuda.Event()
         start.record(self.main)
         for st in self.streams:
             st.wait_event(start)
-        self.i = 0
 
     def next(self):
         """Context manager: run the next layer's update on the next side stream."""
+        if self.streams is None:
+            self._fork()
         st = self.streams[self.i % len(self.streams)]
         self.i += 1
         return torch.cuda.stream(st)
 
     def join(self) -> None:
-        for st in self.streams:
+        for st in self.streams or ():
             ev = torch.cuda.Event()
             ev.record(st)
             self.main.wait_event(ev)

@@ -18,6 +18,8 @@ with zero rows/columns of P and S, which leaves every product unchanged.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 
 from . import _lib as L
@@ -47,26 +49,27 @@ def gemm(M, N, A1, B1, K1, a_layout, b_layout, *, A2=None, B2=None, K2=0, bmask=
     """
     dev = L.require_device(A1, B1, A2, B2, bmask, bias, emask, dw, out, bmask_t)
     dt = A1.dtype
-
-    def _shape(t, want, name):
-        if t is not None and tuple(t.shape) != tuple(want):
-            raise ValueError(f"gemm: {name} has shape {tuple(t.shape)}, expected {tuple(want)}")
-
-    def _op_shape(rows, k, layout):
-        return (rows, k) if layout == L.LAYOUT_K else (k, rows)
-
-    _shape(A1, _op_shape(M, K1, a_layout), "A1")
-    _shape(B1, _op_shape(N, K1, b_layout), "B1")
-    _shape(bmask, _op_shape(N, K1, b_layout), "bmask")
+    # the checks run on every product of a step: inline comparisons, the message built only on a mismatch
+    a_k, b_k = a_layout == L.LAYOUT_K, b_layout == L.LAYOUT_K
+    b1_shape = (N, K1) if b_k else (K1, N)
+    if A1.shape != ((M, K1) if a_k else (K1, M)):
+        _bad_shape("A1", A1, (M, K1) if a_k else (K1, M))
+    if B1.shape != b1_shape:
+        _bad_shape("B1", B1, b1_shape)
+    if bmask is not None and bmask.shape != b1_shape:
+        _bad_shape("bmask", bmask, b1_shape)
     if K2:
         if A2 is None or B2 is None:
             raise ValueError("gemm: K2 > 0 needs A2 and B2")
-        _shape(A2, _op_shape(M, K2, a_layout), "A2")
-        _shape(B2, _op_shape(N, K2, b_layout), "B2")
-    _shape(bias, (N,), "bias")
-    _shape(emask, (M, N), "emask")
-    _shape(dw, (M, N), "dw")
-    _shape(out, (M, N), "out")
+        if A2.shape != ((M, K2) if a_k else (K2, M)):
+            _bad_shape("A2", A2, (M, K2) if a_k else (K2, M))
+        if B2.shape != ((N, K2) if b_k else (K2, N)):
+            _bad_shape("B2", B2, (N, K2) if b_k else (K2, N))
+    if bias is not None and bias.shape != (N,):
+        _bad_shape("bias", bias, (N,))
+    for t, name in ((emask, "emask"), (dw, "dw"), (out, "out")):
+        if t is not None and t.shape != (M, N):
+            _bad_shape(name, t, (M, N))
     bmask_bytes = bmask is not None and bmask.dtype == torch.uint8
     for t in (B1, A2, B2, None if bmask_bytes else bmask, emask, dw):
         if t is not None and t.dtype != dt:
@@ -79,27 +82,34 @@ def gemm(M, N, A1, B1, K1, a_layout, b_layout, *, A2=None, B2=None, K2=0, bmask=
     d.dtype = L.dtype_code(A1)
     d.a_layout, d.b_layout = a_layout, b_layout
     d.M, d.N, d.K1, d.K2 = M, N, K1, K2
-    d.A1, d.B1 = L.ptr(A1), L.ptr(B1)
-    d.lda1 = A1.shape[1]
-    d.ldb1 = B1.shape[1]
+    d.A1, d.B1 = A1.data_ptr(), B1.data_ptr()
+    d.lda1 = K1 if a_k else M
+    d.ldb1 = K1 if b_k else N
     if K2:
-        d.A2, d.B2 = L.ptr(A2), L.ptr(B2)
-        d.lda2, d.ldb2 = A2.shape[1], B2.shape[1]
-    d.bmask = L.ptr(bmask)
-    d.bmask_bytes = int(bmask_bytes)
-    if (bmask_t is not None and bmask_bytes and b_layout == L.LAYOUT_MN and dt == torch.bfloat16
-            and K1 % 16 == 0 and bmask_t.data_ptr() % 16 == 0):
-        _shape(bmask_t, (N, K1), "bmask_t")
-        if bmask_t.dtype != torch.uint8:
-            raise TypeError("gemm: bmask_t must be a uint8 and-mask")
-        d.bmask, d.bmask_kmajor, d.ldbm = L.ptr(bmask_t), 1, K1
-    d.bscale = float(bscale)
-    d.C, d.ldc, d.c_dtype = L.ptr(out), out.shape[1], L.dtype_code(out)
+        d.A2, d.B2 = A2.data_ptr(), B2.data_ptr()
+        d.lda2, d.ldb2 = (K2 if a_k else M), (K2 if b_k else N)
+    if bmask is not None:
+        d.bmask = bmask.data_ptr()
+        d.bmask_bytes = int(bmask_bytes)
+        if (bmask_t is not None and bmask_bytes and not b_k and dt == torch.bfloat16
+                and K1 % 16 == 0 and bmask_t.data_ptr() % 16 == 0):
+            if bmask_t.shape != (N, K1):
+                _bad_shape("bmask_t", bmask_t, (N, K1))
+            if bmask_t.dtype != torch.uint8:
+                raise TypeError("gemm: bmask_t must be a uint8 and-mask")
+            d.bmask, d.bmask_kmajor, d.ldbm = bmask_t.data_ptr(), 1, K1
+    d.bscale = bscale
+    d.C, d.ldc, d.c_dtype = out.data_ptr(), N, L.dtype_code(out)
     if bias is not None:
-        d.bias, d.bias_dtype = L.ptr(bias), L.dtype_code(bias)
-    d.emask, d.dw, d.decay = L.ptr(emask), L.ptr(dw), float(decay)
-    d.accumulate = int(bool(accumulate))
-    ws_bytes = L.lib().sf_gemm_workspace_size(L.byref(d))
+        d.bias, d.bias_dtype = bias.data_ptr(), L.dtype_code(bias)
+    if emask is not None:
+        d.emask = emask.data_ptr()
+    if dw is not None:
+        d.dw, d.decay = dw.data_ptr(), decay
+    if accumulate:
+        d.accumulate = 1
+    ref, lib = ctypes.byref(d), L.lib()
+    ws_bytes = lib.sf_gemm_workspace_size(ref)
     if max_splits is not None and ws_bytes > max_splits * M * N * 4:  # fewer K splits (the big products only)
         ws_bytes = max_splits * M * N * 4 if max_splits > 1 else 0
     ws = None
@@ -107,8 +117,14 @@ def gemm(M, N, A1, B1, K1, a_layout, b_layout, *, A2=None, B2=None, K2=0, bmask=
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         d.workspace, d.workspace_bytes = ws.data_ptr(), ws_bytes
     with _prof.region("sf_gemm", 2.0 * M * N * (K1 + K2), "FLOP", dev):
-        L.check(L.lib().sf_gemm(L.byref(d), L.stream(dev)), "sf_gemm")
+        rc = lib.sf_gemm(ref, L.stream(dev))
+    if rc != L.SF_OK:
+        L.check(rc, "sf_gemm")
     return out
+
+
+def _bad_shape(name, t, want):
+    raise ValueError(f"gemm: {name} has shape {tuple(t.shape)}, expected {tuple(want)}")
 
 
 def mm_nt(A, B, **kw):
@@ -286,25 +302,18 @@ def _opt(t):
     return t.contiguous() if t is not None else None
 
 
-_SIDE: dict = {}
-_CUS: dict = {}
+class _Unrecorded:
+    """Stands in for a Function's ctx when its forward runs outside a graph: nothing is kept."""
+
+    def save_for_backward(self, *tensors):
+        pass
 
 
-def _side_stream(t: torch.Tensor):
-    """A second stream for the weight-gradient products when the two big backward products (dx [T, in] and
-    dW [out, in], 256 x 256 tiles) would each leave compute units idle: running dW beside dx fills them.
-    None when both fill the GPU by themselves (the LLaMA-7B layer shapes) or off the GPU."""
-    if not t.is_cuda:
-        return None
-    dev = t.device.index if t.device.index is not None else torch.cuda.current_device()
-    if dev not in _SIDE:
-        _SIDE[dev] = torch.cuda.Stream(device=dev)  # default priority
-        _CUS[dev] = torch.cuda.get_device_properties(dev).multi_processor_count
-    return _SIDE[dev]
-
-
-def _fills(rows: int, cols: int, dev: int) -> bool:
-    return ((rows + 255) // 256) * ((cols + 255) // 256) >= _CUS[dev]
+def apply_in_backward(fn, *args):
+    """fn.apply(*args) for the gradient Functions (whose backward the Hutchinson probe takes).  In a plain
+    backward pass (no create_graph: grad mode is off) nothing records them, so their forward runs as it is,
+    without the 20 us that an autograd Function's apply costs."""
+    return fn.apply(*args) if torch.is_grad_enabled() else fn.forward(_Unrecorded(), *args)
 
 
 # ---------------------------------------------------------------------------
@@ -323,41 +332,17 @@ class _MaskedLinearBackward(torch.autograd.Function):
         # dx = gy (W.E): the forward's masked weight when it kept one (no weight-scaling factor),
         # else rebuilt with one elementwise pass
         Wm = wm_fwd if wm_fwd is not None else (apply_mask(W, E) if E is not None else W)
-        T, out, inn = gy.shape[0], gy.shape[1], x.shape[1]
-        side = _side_stream(gy)
-        if side is not None:
-            di = gy.device.index if gy.device.index is not None else torch.cuda.current_device()
-            if _fills(T, inn, di) and _fills(out, inn, di):
-                side = None
-        dW = torch.empty(out, inn, dtype=gy.dtype, device=gy.device)  # allocated on the calling stream
-        dS = torch.empty(out, P.shape[0], dtype=gy.dtype, device=gy.device) if has_slorb else None
-        main = torch.cuda.current_stream(gy.device) if side is not None else None
-
-        # beside dx a product needs fewer K splits to fill the compute units dx leaves idle
-        ms = 2 if side is not None else None
-
-        def weight_grads():
-            if decay != 0.0:
-                mm_tn(gy, x, emask=_as_values(E, W.dtype), dw=W, decay=decay, out=dW, max_splits=ms)
-            else:
-                mm_tn(gy, x, out=dW, max_splits=ms)
-            if has_slorb:
-                mm_tn(gy, z, out=dS)
-
-        if side is not None:  # dW and dS beside dz, dx and dP; joined before returning
-            side.wait_stream(main)
-            with torch.cuda.stream(side):
-                weight_grads()
         if has_slorb:
             dx = mm_nn(gy, Wm, A2=dz, B2=P, K2=P.shape[0])
         else:
             dx = mm_nn(gy, Wm)
-        if side is None:
-            weight_grads()
+        if decay != 0.0:
+            dW = mm_tn(gy, x, emask=_as_values(E, W.dtype), dw=W, decay=decay)
+        else:
+            dW = mm_tn(gy, x)
+        dS = mm_tn(gy, z) if has_slorb else None
         db = column_sum(gy, W.dtype) if has_bias else None
         dP = mm_tn(dz, x) if has_slorb else None
-        if side is not None:
-            main.wait_stream(side)
         # W.E stays for the double backward's d/d gy (gdx (W.E)^T), so that product runs unmasked
         ctx.save_for_backward(gy, x, W, P, S, E, z, dz, Wm if E is not None else None)
         del Wm
@@ -388,28 +373,6 @@ class _MaskedLinearBackward(torch.autograd.Function):
         la = _cat_k([t for t in (u, z if g_dS is not None else None) if t is not None], 1)
         lb = _cat_k([t for t, a in ((S, u), (g_dS, g_dS)) if a is not None], 1)
         seg = {"A2": la, "B2": lb, "K2": la.shape[1]} if la is not None else {}
-        # d/dW = (gy^T gdx) . E  (+ decay gdW [E < 0.5]: the SR-STE term decay W [E < 0.5] of dW is
-        # elementwise in W, legacy/sparse_modeling.py:123-125), beside the two products below when
-        # they leave compute units idle (as in forward())
-        gW = None
-        side = _side_stream(gy) if g_dx is not None else None
-        if side is not None:
-            di = gy.device.index if gy.device.index is not None else torch.cuda.current_device()
-            if _fills(T, x.shape[1], di) and _fills(out, x.shape[1], di):
-                side = None
-        if g_dx is not None:
-            gW = torch.empty(out, x.shape[1], dtype=gy.dtype, device=gy.device)
-        main = torch.cuda.current_stream(gy.device) if side is not None else None
-
-        def weight_grad():
-            if g_dx is not None:
-                mm_tn(gy, g_dx, emask=_as_values(E, W.dtype), out=gW, max_splits=2 if side is not None else None)
-            return decay_term(g_dW, E, ctx.decay, out=gW) if ctx.decay != 0.0 and g_dW is not None else gW
-
-        if side is not None:
-            side.wait_stream(main)
-            with torch.cuda.stream(side):
-                weight_grad()
         ggy = None
         if g_dx is not None:
             ggy = mm_nt(g_dx, Wm if Wm is not None else W, bias=g_db, **seg)
@@ -431,10 +394,11 @@ class _MaskedLinearBackward(torch.autograd.Function):
             gx = mm_nn(gy, g_dW, **({"A2": ra, "B2": rb, "K2": ra.shape[1]} if ra is not None else {}))
         elif ra is not None:
             gx = mm_nn(ra, rb)
-        if side is None:
-            gW = weight_grad()
-        else:
-            main.wait_stream(side)
+        # d/dW = (gy^T gdx) . E  (+ decay gdW [E < 0.5]: the SR-STE term decay W [E < 0.5] of dW is
+        # elementwise in W, legacy/sparse_modeling.py:123-125)
+        gW = mm_tn(gy, g_dx, emask=_as_values(E, W.dtype)) if g_dx is not None else None
+        if ctx.decay != 0.0 and g_dW is not None:
+            gW = decay_term(g_dW, E, ctx.decay, out=gW)
         # d/dP = dz^T gdx + (gy gdS)^T x ;  d/dS = gy^T (gdx P^T + x gdP^T)
         gP = gS = None
         if ctx.has_slorb:
@@ -484,7 +448,8 @@ class _MaskedLinear(torch.autograd.Function):
     def backward(ctx, gy):
         x2, W, P, S, E, z, wm = ctx.saved_tensors
         gy = gy.contiguous().to(W.dtype)
-        dx, dW, db, dP, dS = _MaskedLinearBackward.apply(gy, x2, W, P, S, E, ctx.decay, ctx.has_bias, z, wm)
+        dx, dW, db, dP, dS = apply_in_backward(_MaskedLinearBackward, gy, x2, W, P, S, E, ctx.decay, ctx.has_bias, z,
+                                               wm)
         del wm
         return dx, dW, db, dP, dS, None, None, None, None
 

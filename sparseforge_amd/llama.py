@@ -43,6 +43,7 @@ from torch.nn import functional as F
 
 from . import _lib as L
 from . import profiling as _prof
+from .linear import apply_in_backward
 from .sparse_modeling import SparseLinear, SparseLinearConfig
 
 
@@ -125,7 +126,7 @@ class _RMSNorm(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gy):
         x2, w, rstd = ctx.saved_tensors
-        gx, gw = _RMSNormGrad.apply(gy.to(x2.dtype), x2, w, rstd)
+        gx, gw = apply_in_backward(_RMSNormGrad, gy.to(x2.dtype), x2, w, rstd)
         return gx, gw, None
 
 
@@ -328,7 +329,7 @@ class _CausalSoftmax(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gp):
         x, = ctx.saved_tensors
-        return _CausalSoftmaxGrad.apply(gp.to(x.dtype).contiguous(), x)
+        return apply_in_backward(_CausalSoftmaxGrad, gp.to(x.dtype).contiguous(), x)
 
 
 class _CausalSoftmaxGrad(torch.autograd.Function):
@@ -593,7 +594,7 @@ class _SwiGLU(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gy):
         g, u = ctx.saved_tensors
-        return _SwiGLUGrad.apply(_aligned(gy.to(g.dtype)), g, u)
+        return apply_in_backward(_SwiGLUGrad, _aligned(gy.to(g.dtype)), g, u)
 
 
 class _SwiGLUGrad(torch.autograd.Function):

@@ -88,15 +88,41 @@ def kernel_timer():
         _active = None
 
 
-@contextlib.contextmanager
+class _Region:
+    __slots__ = ("timer", "rec", "device")
+
+    def __init__(self, timer: KernelTimer, rec: _Rec, device: torch.device):
+        self.timer, self.rec, self.device = timer, rec, device
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        self.timer.end(self.rec, self.device)
+        return False
+
+
+class _NoRegion:
+    __slots__ = ()
+
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_NO_REGION = _NoRegion()
+
+
+def active() -> bool:
+    """Whether a KernelTimer is active (callers skip adding up a region's work otherwise)."""
+    return _active is not None
+
+
 def region(name: str, work: float, unit: str, device: torch.device):
     """Bracket one C-ABI launch; a no-op unless a KernelTimer is active."""
     t = _active
     if t is None:
-        yield
-        return
-    rec = t.begin(name, work, unit, device)
-    try:
-        yield
-    finally:
-        t.end(rec, device)
+        return _NO_REGION
+    return _Region(t, t.begin(name, work, unit, device), device)

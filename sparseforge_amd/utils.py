@@ -167,7 +167,8 @@ def calculate_model_mask(model, step=0, lambda_mid: float = 0.0):
         q = float(m._effective_sparsity(step)) if p.gate == L.GATE_UNSTRUCTURED else 0.0
         shape_free = L.MaskParams.from_buffer_copy(p)
         shape_free.rows = shape_free.cols = 0
-        key = (ops.device(), tuple(ops.dt(t) if t is not None else -1
+        dev = ops.device()
+        key = (dev, tuple(ops.dt(t) if t is not None else -1
                                    for t in (ops.weight, ops.hessian, ops.aux, ops.mask, ops.frozen)),
                bytes(shape_free), q)
         # the tau sample's seed, drawn here so every layer (staged or batched) draws in module order, as one
@@ -176,7 +177,7 @@ def calculate_model_mask(model, step=0, lambda_mid: float = 0.0):
         idx = None
         if seed is not None:
             idx = (m._sample_size(ops.weight.numel()), ops.weight.numel(), seed)
-            draws.setdefault((ops.device(), idx[0]), []).append(idx)
+            draws.setdefault((dev, idx[0]), []).append(idx)
         batches.setdefault(key, []).append([m, ops, p, idx])
     for (dev, size), lists in draws.items():
         rows = draw_samples(size, [n for _, n, _ in lists], [s for _, _, s in lists], dev)
