@@ -308,6 +308,9 @@ class _Unrecorded:
     def save_for_backward(self, *tensors):
         pass
 
+    def set_materialize_grads(self, value):
+        pass
+
 
 def apply_in_backward(fn, *args):
     """fn.apply(*args) for the gradient Functions (whose backward the Hutchinson probe takes).  In a plain
@@ -343,6 +346,9 @@ class _MaskedLinearBackward(torch.autograd.Function):
         dS = mm_tn(gy, z) if has_slorb else None
         db = column_sum(gy, W.dtype) if has_bias else None
         dP = mm_tn(dz, x) if has_slorb else None
+        # outputs that no derivative reaches (a probe of the weight gradients leaves dP, dS and db out) come to
+        # backward() as None and cost no product; zeros made for them were multiplied through six products
+        ctx.set_materialize_grads(False)
         # W.E stays for the double backward's d/d gy (gdx (W.E)^T), so that product runs unmasked
         ctx.save_for_backward(gy, x, W, P, S, E, z, dz, Wm if E is not None else None)
         del Wm
@@ -411,6 +417,9 @@ class _MaskedLinearBackward(torch.autograd.Function):
                 gP = mm_tn(w, x)
             if u is not None:
                 gS = mm_tn(gy, u)
+            gP, gS = (torch.zeros_like(t) if g is None else g for g, t in ((gP, P), (gS, S)))
+        # a derivative that is identically zero is still a tensor (callers without allow_unused)
+        gx, gW = (torch.zeros_like(t) if g is None else g for g, t in ((gx, x), (gW, W)))
         return ggy, gx, gW, gP, gS, None, None, None, None, None
 
 

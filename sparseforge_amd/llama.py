@@ -142,6 +142,7 @@ class _RMSNormGrad(torch.autograd.Function):
             L.check(L.lib().sf_rmsnorm_backward(L.ptr(x2), L.ptr(w), L.ptr(gy), L.ptr(rstd), L.dtype_code(x2), rows,
                                                 D, L.ptr(gx), L.ptr(gw), L.ptr(ws), ws.numel(), L.stream(dev)),
                     "sf_rmsnorm_backward")
+        ctx.set_materialize_grads(False)  # an output that no derivative reaches comes to backward() as None
         ctx.save_for_backward(gy, x2, w, rstd)
         return gx, gw
 
@@ -604,6 +605,7 @@ class _SwiGLUGrad(torch.autograd.Function):
         gg, gu = torch.empty_like(g), torch.empty_like(g)
         _sg_launch("sf_swiglu_backward", 5 * g.numel() * g.element_size(), dev, L.ptr(g), L.ptr(u), L.ptr(gy),
                    L.dtype_code(g), g.numel(), L.ptr(gg), L.ptr(gu))
+        ctx.set_materialize_grads(False)
         ctx.save_for_backward(gy, g, u)
         return gg, gu
 

@@ -193,3 +193,25 @@ def test_multi_tensor_update_equals_single_updates(cuda_device, hdt, vdt):
         utils.hutchinson_update_(H, hvp, beta, seed=seed)
     for (a, *_), (b, *_) in zip(items_a, items_b):
         assert torch.equal(a, b)
+
+
+def test_probe_of_a_loss_linear_in_the_output(cuda_device):
+    """Outputs of the gradient that no derivative reaches are left out of the products, and derivatives that are
+    identically zero still come as zeros: the loss is linear in y, so nothing second-order depends on the weight."""
+    from sparseforge_amd import sparse_modeling as sm
+
+    cfg = sm.SparseLinearConfig(mask_type="unstructured", hard_mask_type="nm_2_4", SLoRB=True, SLoRB_k=16,
+                                trainable_projection=True)
+    lin = sm.SparseLinear(128, 96, sparselinear_config=cfg, bias=True).to(cuda_device)
+    with torch.no_grad():
+        lin.x_proj.normal_()
+        lin.SLoRB_Weight.normal_()
+    x = torch.randn(64, 128, device=cuda_device, requires_grad=True)
+    loss = (lin(x) * torch.randn(64, 96, device=cuda_device)).sum()
+    params = [lin.weight, lin.x_proj, lin.SLoRB_Weight, x]
+    for k in range(3):  # a probe of dW, dP, dS alone: no derivative of the others
+        g, = torch.autograd.grad(loss, params[k:k + 1], create_graph=True)
+        hv = torch.autograd.grad((g * torch.randn_like(g)).sum(), params, retain_graph=True)
+        assert all(torch.isfinite(h).all() for h in hv)
+        assert not hv[0].any()  # d2 / dW . : dW, dP and dS do not contain W
+        assert bool(hv[3].any())
