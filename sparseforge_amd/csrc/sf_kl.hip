@@ -23,7 +23,6 @@
 namespace sf {
 namespace {
 
-constexpr int kKlBlock = 256;
 constexpr int kKlFinalBlock = 1024;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kKlU = 4;  // slices of a row a thread loads before using them (forward)
@@ -178,34 +177,57 @@ __device__ __forceinline__ void kl_slice(KlAcc& acc, bool& bad, float (&a)[8], f
   }
 }
 
-// One workgroup per token row; thread t takes slices t, t + 256, ... in order.
-// VEC (vocab % 8 == 0, 16-byte aligned rows): every slice is whole and a
-// thread's next two slices of both rows are loaded before either is used.
-template <int DT, bool VEC>
-__global__ void __launch_bounds__(kKlBlock) kl_rows_kernel(const void* __restrict__ s, const void* __restrict__ t,
+// Elements of a row before its first 16-byte boundary (16-byte aligned tensors: the same for all of a row's tensors).
+template <int DT>
+__device__ __forceinline__ int kl_head(int64_t base, int64_t vocab) {
+  constexpr int PER = DT == SF_DTYPE_F32 ? 4 : 8;  // elements per 16 bytes
+  const int h = static_cast<int>((PER - base % PER) % PER);
+  return h < vocab ? h : static_cast<int>(vocab);
+}
+
+// One workgroup per token row; thread t takes slices t, t + BLK, ... in order.
+// VEC (16-byte aligned tensors): the slices start at the row's first 16-byte
+// boundary, so every one is whole and vector-loaded whatever the vocabulary, and
+// a thread's next four slices of both rows are loaded before any is used; the
+// last thread takes the up to 7 elements before them, the one before it those
+// after.  (An odd vocabulary took the element-by-element path: loss and gradient
+// of [1024, 50257] bf16 288 us, 120 here; f32 468 and 245.)
+// BLK: 1024 threads a row when there are too few rows to fill the GPU at 256.
+template <int DT, bool VEC, int BLK>
+__global__ void __launch_bounds__(BLK) kl_rows_kernel(const void* __restrict__ s, const void* __restrict__ t,
                                                            int64_t vocab, float inv_t, double* __restrict__ lse,
                                                            double* __restrict__ row_kl, int* __restrict__ row_nan) {
   const int64_t r = blockIdx.x, base = r * vocab;
   KlAcc acc{-INFINITY, 0.0f, -INFINITY, 0.0f, 0.0f};
   bool bad = false;
   if constexpr (VEC) {
-    const int64_t slices = vocab / 8, step = blockDim.x;
+    const int head = kl_head<DT>(base, vocab);
+    const int64_t slices = (vocab - head) / 8, step = BLK, b0 = base + head;
     int64_t c = threadIdx.x;
     for (; c + (kKlU - 1) * step < slices; c += kKlU * step) {
       float a[kKlU][8], b[kKlU][8];
 #pragma unroll
       for (int u = 0; u < kKlU; ++u) {
-        load8<DT>(s, base + 8 * (c + u * step), 8, true, a[u]);
-        load8<DT>(t, base + 8 * (c + u * step), 8, true, b[u]);
+        load8<DT>(s, b0 + 8 * (c + u * step), 8, true, a[u]);
+        load8<DT>(t, b0 + 8 * (c + u * step), 8, true, b[u]);
       }
 #pragma unroll
       for (int u = 0; u < kKlU; ++u) kl_slice(acc, bad, a[u], b[u], 8, inv_t);
     }
     for (; c < slices; c += step) {
-      float a0[8], b0[8];
-      load8<DT>(s, base + 8 * c, 8, true, a0);
-      load8<DT>(t, base + 8 * c, 8, true, b0);
-      kl_slice(acc, bad, a0, b0, 8, inv_t);
+      float x[8], y[8];
+      load8<DT>(s, b0 + 8 * c, 8, true, x);
+      load8<DT>(t, b0 + 8 * c, 8, true, y);
+      kl_slice(acc, bad, x, y, 8, inv_t);
+    }
+    const int64_t done = head + 8 * slices;
+    const int n = threadIdx.x == BLK - 1 ? head : (threadIdx.x == BLK - 2 ? static_cast<int>(vocab - done) : 0);
+    if (n > 0) {
+      const int64_t at = base + (threadIdx.x == BLK - 1 ? 0 : done);
+      float x[8], y[8];
+      load8<DT>(s, at, n, false, x);
+      load8<DT>(t, at, n, false, y);
+      kl_slice(acc, bad, x, y, n, inv_t);
     }
   } else {
     for (int64_t j0 = threadIdx.x * 8; j0 < vocab; j0 += 8 * (int64_t)blockDim.x) {
@@ -219,8 +241,8 @@ __global__ void __launch_bounds__(kKlBlock) kl_rows_kernel(const void* __restric
   int nan = bad;
   for (int off = 32; off > 0; off >>= 1) acc = kl_merge(acc, kl_shfl_xor(acc, off));
   for (int off = 32; off > 0; off >>= 1) nan |= __shfl_xor(nan, off, 64);
-  __shared__ KlAcc part[kKlBlock / 64];
-  __shared__ int pnan[kKlBlock / 64];
+  __shared__ KlAcc part[BLK / 64];
+  __shared__ int pnan[BLK / 64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   if (lane == 0) {
     part[wv] = acc;
@@ -230,7 +252,7 @@ __global__ void __launch_bounds__(kKlBlock) kl_rows_kernel(const void* __restric
   if (threadIdx.x == 0) {
     KlAcc x = part[0];
     int nn = pnan[0];
-    for (int w = 1; w < (int)(blockDim.x / 64); ++w) {
+    for (int w = 1; w < BLK / 64; ++w) {
       x = kl_merge(x, part[w]);
       nn |= pnan[w];
     }
@@ -315,8 +337,8 @@ __device__ __forceinline__ float kl_grad1(float a, float b, float inv_t, double 
 
 // One workgroup per token row, slices as in kl_rows_kernel (VEC: kKlBwdU
 // slices' loads in flight per thread); rows whose chunk was dropped get zeros.
-template <int DT, bool VEC>
-__global__ void __launch_bounds__(kKlBlock) kl_backward_kernel(const void* __restrict__ s, const void* __restrict__ t,
+template <int DT, bool VEC, int BLK>
+__global__ void __launch_bounds__(BLK) kl_backward_kernel(const void* __restrict__ s, const void* __restrict__ t,
                                                                int64_t vocab, float inv_t,
                                                                const double* __restrict__ lse,
                                                                const float* __restrict__ row_scale,
@@ -326,10 +348,14 @@ __global__ void __launch_bounds__(kKlBlock) kl_backward_kernel(const void* __res
   const float factor = row_scale[r] * load_as_f32(gout, 0, gout_dtype);
   const double ls = lse[2 * r], lt = lse[2 * r + 1];
   if constexpr (VEC) {
-    const int64_t slices = vocab / 8, step = blockDim.x;
+    const int head = kl_head<DT>(base, vocab);
+    const int64_t slices = (vocab - head) / 8, step = BLK, b0 = base + head, done = head + 8 * slices;
+    const int n = threadIdx.x == BLK - 1 ? head : (threadIdx.x == BLK - 2 ? static_cast<int>(vocab - done) : 0);
+    const int64_t at = base + (threadIdx.x == BLK - 1 ? 0 : done);  // this thread's odd elements (n of them)
     if (factor == 0.0f) {
       const float z[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-      for (int64_t c = threadIdx.x; c < slices; c += step) store8<DT>(gs, base + 8 * c, 8, true, z);
+      for (int64_t c = threadIdx.x; c < slices; c += step) store8<DT>(gs, b0 + 8 * c, 8, true, z);
+      if (n > 0) store8<DT>(gs, at, n, false, z);
       return;
     }
     int64_t c = threadIdx.x;
@@ -337,23 +363,31 @@ __global__ void __launch_bounds__(kKlBlock) kl_backward_kernel(const void* __res
       float a[kKlBwdU][8], b[kKlBwdU][8];
 #pragma unroll
       for (int u = 0; u < kKlBwdU; ++u) {
-        load8<DT>(s, base + 8 * (c + u * step), 8, true, a[u]);
-        load8<DT>(t, base + 8 * (c + u * step), 8, true, b[u]);
+        load8<DT>(s, b0 + 8 * (c + u * step), 8, true, a[u]);
+        load8<DT>(t, b0 + 8 * (c + u * step), 8, true, b[u]);
       }
 #pragma unroll
       for (int u = 0; u < kKlBwdU; ++u) {
 #pragma unroll
         for (int k = 0; k < 8; ++k) a[u][k] = kl_grad1(a[u][k], b[u][k], inv_t, ls, lt, factor);
-        store8<DT>(gs, base + 8 * (c + u * step), 8, true, a[u]);
+        store8<DT>(gs, b0 + 8 * (c + u * step), 8, true, a[u]);
       }
     }
     for (; c < slices; c += step) {
-      float a0[8], b0[8];
-      load8<DT>(s, base + 8 * c, 8, true, a0);
-      load8<DT>(t, base + 8 * c, 8, true, b0);
+      float x[8], y[8];
+      load8<DT>(s, b0 + 8 * c, 8, true, x);
+      load8<DT>(t, b0 + 8 * c, 8, true, y);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) a0[k] = kl_grad1(a0[k], b0[k], inv_t, ls, lt, factor);
-      store8<DT>(gs, base + 8 * c, 8, true, a0);
+      for (int k = 0; k < 8; ++k) x[k] = kl_grad1(x[k], y[k], inv_t, ls, lt, factor);
+      store8<DT>(gs, b0 + 8 * c, 8, true, x);
+    }
+    if (n > 0) {
+      float x[8], y[8];
+      load8<DT>(s, at, n, false, x);
+      load8<DT>(t, at, n, false, y);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) x[k] = kl_grad1(x[k], y[k], inv_t, ls, lt, factor);
+      store8<DT>(gs, at, n, false, x);
     }
   } else {
     for (int64_t j0 = threadIdx.x * 8; j0 < vocab; j0 += 8 * (int64_t)blockDim.x) {
@@ -369,13 +403,14 @@ __global__ void __launch_bounds__(kKlBlock) kl_backward_kernel(const void* __res
 }
 
 bool kl_dtype_ok(int d) { return d == SF_DTYPE_F32 || d == SF_DTYPE_BF16; }
-bool kl_vec_ok(int64_t vocab, int dtype, std::initializer_list<const void*> ptrs) {
-  if (vocab % 8 != 0) return false;
+bool kl_vec_ok(std::initializer_list<const void*> ptrs) {
   for (const void* p : ptrs)
     if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return false;
-  (void)dtype;
   return true;
 }
+// Rows up to one per CU leave too little in flight at 256 threads: 1024 threads a row (183 x 128256 bf16 forward 38 ->
+// 31 us, backward 47 -> 31; 76 x 32000 f32 15 and 16 -> 15 and 11).  600 rows are better at 256 (32 against 47 us).
+constexpr int64_t kKlFewRows = 257;
 size_t a256(size_t b) { return (b + 255) / 256 * 256; }
 }  // namespace
 }  // namespace sf
@@ -403,11 +438,16 @@ extern "C" int sf_kl_forward(const void* student, const void* teacher, int dtype
   double* row_kl = static_cast<double*>(workspace);
   int* row_nan = reinterpret_cast<int*>(static_cast<char*>(workspace) + a256(static_cast<size_t>(rows) * 8));
   const float inv_t = static_cast<float>(1.0 / static_cast<double>(temperature));
-  const bool vec = kl_vec_ok(vocab, dtype, {student, teacher});
+  const bool vec = kl_vec_ok({student, teacher});
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 grid(static_cast<unsigned>(rows));
-#define SF_KL_ROWS(DT, V) kl_rows_kernel<DT, V><<<grid, kKlBlock, 0, st>>>(student, teacher, vocab, inv_t, row_lse, \
-                                                                          row_kl, row_nan)
+#define SF_KL_ROWS(DT, V)                                                                                              \
+  do {                                                                                                                 \
+    if (rows < kKlFewRows)                                                                                             \
+      kl_rows_kernel<DT, V, 1024><<<grid, 1024, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_kl, row_nan);    \
+    else                                                                                                               \
+      kl_rows_kernel<DT, V, 256><<<grid, 256, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_kl, row_nan);      \
+  } while (0)
   if (dtype == SF_DTYPE_F32) {
     if (vec)
       SF_KL_ROWS(SF_DTYPE_F32, true);
@@ -435,12 +475,18 @@ extern "C" int sf_kl_backward(const void* student, const void* teacher, int dtyp
   SF_CHECK_ARG(temperature > 0.0f, "temperature must be positive");
   SF_CHECK_ARG(rows < (1ll << 31), "more than 2^31 token rows");
   const float inv_t = static_cast<float>(1.0 / static_cast<double>(temperature));
-  const bool vec = kl_vec_ok(vocab, dtype, {student, teacher, grad_student});
+  const bool vec = kl_vec_ok({student, teacher, grad_student});
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 grid(static_cast<unsigned>(rows));
-#define SF_KL_BWD(DT, V)                                                                                    \
-  kl_backward_kernel<DT, V><<<grid, kKlBlock, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_scale, grad_out, \
-                                                       grad_out_dtype, grad_student)
+#define SF_KL_BWD(DT, V)                                                                                          \
+  do {                                                                                                            \
+    if (rows < kKlFewRows)                                                                                        \
+      kl_backward_kernel<DT, V, 1024><<<grid, 1024, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_scale,  \
+                                                             grad_out, grad_out_dtype, grad_student);             \
+    else                                                                                                          \
+      kl_backward_kernel<DT, V, 256><<<grid, 256, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_scale,    \
+                                                           grad_out, grad_out_dtype, grad_student);               \
+  } while (0)
   if (dtype == SF_DTYPE_F32) {
     if (vec)
       SF_KL_BWD(SF_DTYPE_F32, true);
