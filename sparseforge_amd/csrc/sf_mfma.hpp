@@ -249,6 +249,11 @@ __device__ __forceinline__ void store_c8(const GemmArgs& g, int64_t row, int64_t
 // C = epilogue(sum of the K splits' partials) (sf_splitk.hip).
 int launch_splitk_reduce(const GemmArgs& g, int elem_dtype, hipStream_t st, const char* what);
 
+// The bf16 product of dense, unmasked operands with a side of C of at most 64 (sf_gemm_skinny.hip): its workspace for
+// K-split partials (often none), and the launch.
+size_t gemm_skinny_workspace(int64_t M, int64_t N, int64_t K, int a_layout, int b_layout);
+int launch_gemm_skinny(GemmArgs g, int a_layout, int b_layout, void* workspace, size_t workspace_bytes, hipStream_t st);
+
 // The bf16 product of dense, unmasked operands on 128 x 128 tiles (sf_gemm_mid.hip): K splits it would take (0: the
 // 256 x 256 tiles are the better choice), and its launch.
 int gemm_mid_splits(int64_t M, int64_t N, int64_t K, int max_splits, int big_splits);
