@@ -14,8 +14,8 @@
 // of a row, so C leaves with its epilogue and results do not vary between runs.  K is
 // split over workgroups as well where few tiles meet a long K (skinny_plan).
 // Kernel + reduce at rank 64, z / dP, before (128 x 64 tiles, K split over
-// workgroups) and here: 2048 tokens 2048 -> 2048 15.5 / 15.8 us and 8.6 / 7.8; 4096
-// tokens 15.5 / 16.9 and 9.3 / 12.7; 8192 tokens 4096 -> 11008 19.5 / 22 and 20 / 21,
+// workgroups) and here: 2048 tokens 2048 -> 2048 15.5 / 15.8 us and 8.5 / 8.3; 4096
+// tokens 15.5 / 16.9 and 9.3 / 13; 8192 tokens 4096 -> 11008 19.5 / 22 and 20 / 21,
 // its dS 49 and 37 (what the long operand takes to read).
 #include <type_traits>
 

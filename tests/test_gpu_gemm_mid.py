@@ -15,7 +15,7 @@ def _mk(g, dev, *shape):
 
 @pytest.mark.parametrize("M,N,K", [
     (72, 72, 8), (128, 128, 64), (136, 72, 72), (256, 264, 1000), (1024, 2048, 2048), (520, 2056, 200),
-    (1000, 704, 1952), (2048, 2048, 4096), (4096, 2048, 520),
+    (1000, 704, 1952), (2048, 2048, 4096), (4096, 2048, 520), (2184, 2056, 8), (2184, 2056, 136),
 ])
 @pytest.mark.parametrize("layout", ["nt", "nn", "tn"])
 def test_layouts(cuda_device, M, N, K, layout):
