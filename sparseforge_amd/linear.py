@@ -21,6 +21,7 @@ from __future__ import annotations
 import ctypes
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib as L
 from . import kernels as K
@@ -312,11 +313,18 @@ class _Unrecorded:
         pass
 
 
+def plain_backward() -> bool:
+    """Whether a backward pass runs with nothing that looks into it: no create_graph (grad mode is on then), no
+    functorch transform (torch.func, vmap) and no forward-mode level, which a direct call would pass by."""
+    return not (torch.is_grad_enabled() or forward_ad._current_level >= 0
+                or torch._C._are_functorch_transforms_active())
+
+
 def apply_in_backward(fn, *args):
     """fn.apply(*args) for the gradient Functions (whose backward the Hutchinson probe takes).  In a plain
-    backward pass (no create_graph: grad mode is off) nothing records them, so their forward runs as it is,
-    without the 20 us that an autograd Function's apply costs."""
-    return fn.apply(*args) if torch.is_grad_enabled() else fn.forward(_Unrecorded(), *args)
+    backward pass nothing records them, so their forward runs as it is, without the 20 us that an autograd
+    Function's apply costs; elsewhere apply records, transforms or refuses them."""
+    return fn.forward(_Unrecorded(), *args) if plain_backward() else fn.apply(*args)
 
 
 # ---------------------------------------------------------------------------

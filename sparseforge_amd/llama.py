@@ -43,7 +43,7 @@ from torch.nn import functional as F
 
 from . import _lib as L
 from . import profiling as _prof
-from .linear import apply_in_backward
+from .linear import apply_in_backward, plain_backward
 from .sparse_modeling import SparseLinear, SparseLinearConfig
 
 
@@ -498,10 +498,12 @@ class _FusedAttention(torch.autograd.Function):
     @staticmethod
     def backward(ctx, go):
         q, k, v, cos, sin, qr, kr, out, lse = ctx.saved_tensors
-        if torch.is_grad_enabled():  # create_graph
+        if not plain_backward():  # create_graph, or a transform that the passes' own Functions take or refuse
             wanted = [t for t, n in zip((q, k, v), ctx.needs_input_grad) if n]
-            grads = iter(torch.autograd.grad(_causal_attention_device(q, k, v, cos, sin), wanted, go,
-                                             create_graph=True))
+            create_graph = torch.is_grad_enabled()
+            with torch.enable_grad():
+                o = _causal_attention_device(q, k, v, cos, sin)
+            grads = iter(torch.autograd.grad(o, wanted, go, create_graph=create_graph))
             return (*(next(grads) if n else None for n in ctx.needs_input_grad[:3]), None, None)
         dev = q.device
         B, S, H, D = q.shape
