@@ -17,6 +17,7 @@
 //   dL/ds = g (T / tokens) (q - p) [-100 <= s <= 100].
 
 #include <initializer_list>
+#include <type_traits>
 
 #include "sf_common.hpp"
 
@@ -193,7 +194,11 @@ __device__ __forceinline__ int kl_head(int64_t base, int64_t vocab) {
 // after.  (An odd vocabulary took the element-by-element path: loss and gradient
 // of [1024, 50257] bf16 288 us, 120 here; f32 468 and 245.)
 // BLK: 1024 threads a row when there are too few rows to fill the GPU at 256.
-template <int DT, bool VEC, int BLK>
+// ODD: the vocabulary is no multiple of 8; without it every row starts on a boundary and is whole slices.
+// The step between a thread's slices is read from the launch where it is not ODD: as a constant it lets the
+// compiler keep fewer loads in flight (f32 4096 x 32000, loss and gradient: 586 us against 539); with the odd
+// elements the constant is the better one (f32 2600 x 50257 623 against 659).
+template <int DT, bool VEC, bool ODD, int BLK>
 __global__ void __launch_bounds__(BLK) kl_rows_kernel(const void* __restrict__ s, const void* __restrict__ t,
                                                            int64_t vocab, float inv_t, double* __restrict__ lse,
                                                            double* __restrict__ row_kl, int* __restrict__ row_nan) {
@@ -201,8 +206,8 @@ __global__ void __launch_bounds__(BLK) kl_rows_kernel(const void* __restrict__ s
   KlAcc acc{-INFINITY, 0.0f, -INFINITY, 0.0f, 0.0f};
   bool bad = false;
   if constexpr (VEC) {
-    const int head = kl_head<DT>(base, vocab);
-    const int64_t slices = (vocab - head) / 8, step = BLK, b0 = base + head;
+    const int head = ODD ? kl_head<DT>(base, vocab) : 0;
+    const int64_t slices = (vocab - head) / 8, step = ODD ? BLK : blockDim.x, b0 = base + head;
     int64_t c = threadIdx.x;
     for (; c + (kKlU - 1) * step < slices; c += kKlU * step) {
       float a[kKlU][8], b[kKlU][8];
@@ -220,14 +225,16 @@ __global__ void __launch_bounds__(BLK) kl_rows_kernel(const void* __restrict__ s
       load8<DT>(t, b0 + 8 * c, 8, true, y);
       kl_slice(acc, bad, x, y, 8, inv_t);
     }
-    const int64_t done = head + 8 * slices;
-    const int n = threadIdx.x == BLK - 1 ? head : (threadIdx.x == BLK - 2 ? static_cast<int>(vocab - done) : 0);
-    if (n > 0) {
-      const int64_t at = base + (threadIdx.x == BLK - 1 ? 0 : done);
-      float x[8], y[8];
-      load8<DT>(s, at, n, false, x);
-      load8<DT>(t, at, n, false, y);
-      kl_slice(acc, bad, x, y, n, inv_t);
+    if constexpr (ODD) {
+      const int64_t done = head + 8 * slices;
+      const int n = threadIdx.x == BLK - 1 ? head : (threadIdx.x == BLK - 2 ? static_cast<int>(vocab - done) : 0);
+      if (n > 0) {
+        const int64_t at = base + (threadIdx.x == BLK - 1 ? 0 : done);
+        float x[8], y[8];
+        load8<DT>(s, at, n, false, x);
+        load8<DT>(t, at, n, false, y);
+        kl_slice(acc, bad, x, y, n, inv_t);
+      }
     }
   } else {
     for (int64_t j0 = threadIdx.x * 8; j0 < vocab; j0 += 8 * (int64_t)blockDim.x) {
@@ -337,7 +344,7 @@ __device__ __forceinline__ float kl_grad1(float a, float b, float inv_t, double 
 
 // One workgroup per token row, slices as in kl_rows_kernel (VEC: kKlBwdU
 // slices' loads in flight per thread); rows whose chunk was dropped get zeros.
-template <int DT, bool VEC, int BLK>
+template <int DT, bool VEC, bool ODD, int BLK>
 __global__ void __launch_bounds__(BLK) kl_backward_kernel(const void* __restrict__ s, const void* __restrict__ t,
                                                                int64_t vocab, float inv_t,
                                                                const double* __restrict__ lse,
@@ -348,9 +355,9 @@ __global__ void __launch_bounds__(BLK) kl_backward_kernel(const void* __restrict
   const float factor = row_scale[r] * load_as_f32(gout, 0, gout_dtype);
   const double ls = lse[2 * r], lt = lse[2 * r + 1];
   if constexpr (VEC) {
-    const int head = kl_head<DT>(base, vocab);
-    const int64_t slices = (vocab - head) / 8, step = BLK, b0 = base + head, done = head + 8 * slices;
-    const int n = threadIdx.x == BLK - 1 ? head : (threadIdx.x == BLK - 2 ? static_cast<int>(vocab - done) : 0);
+    const int head = ODD ? kl_head<DT>(base, vocab) : 0;
+    const int64_t slices = (vocab - head) / 8, step = ODD ? BLK : blockDim.x, b0 = base + head, done = head + 8 * slices;
+    const int n = !ODD ? 0 : threadIdx.x == BLK - 1 ? head : threadIdx.x == BLK - 2 ? static_cast<int>(vocab - done) : 0;
     const int64_t at = base + (threadIdx.x == BLK - 1 ? 0 : done);  // this thread's odd elements (n of them)
     if (factor == 0.0f) {
       const float z[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
@@ -411,6 +418,22 @@ bool kl_vec_ok(std::initializer_list<const void*> ptrs) {
 // Rows up to one per CU leave too little in flight at 256 threads: 1024 threads a row (183 x 128256 bf16 forward 38 ->
 // 31 us, backward 47 -> 31; 76 x 32000 f32 15 and 16 -> 15 and 11).  600 rows are better at 256 (32 against 47 us).
 constexpr int64_t kKlFewRows = 257;
+// launch(data type, vector path, odd vocabulary) with the three as constants.
+template <typename F>
+void kl_dispatch(int dtype, bool vec, bool odd, F&& launch) {
+  auto with = [&](auto dt) {
+    if (!vec)
+      launch(dt, std::false_type{}, std::false_type{});
+    else if (odd)
+      launch(dt, std::true_type{}, std::true_type{});
+    else
+      launch(dt, std::true_type{}, std::false_type{});
+  };
+  if (dtype == SF_DTYPE_F32)
+    with(std::integral_constant<int, SF_DTYPE_F32>{});
+  else
+    with(std::integral_constant<int, SF_DTYPE_BF16>{});
+}
 size_t a256(size_t b) { return (b + 255) / 256 * 256; }
 }  // namespace
 }  // namespace sf
@@ -441,25 +464,16 @@ extern "C" int sf_kl_forward(const void* student, const void* teacher, int dtype
   const bool vec = kl_vec_ok({student, teacher});
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 grid(static_cast<unsigned>(rows));
-#define SF_KL_ROWS(DT, V)                                                                                              \
-  do {                                                                                                                 \
-    if (rows < kKlFewRows)                                                                                             \
-      kl_rows_kernel<DT, V, 1024><<<grid, 1024, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_kl, row_nan);    \
-    else                                                                                                               \
-      kl_rows_kernel<DT, V, 256><<<grid, 256, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_kl, row_nan);      \
-  } while (0)
-  if (dtype == SF_DTYPE_F32) {
-    if (vec)
-      SF_KL_ROWS(SF_DTYPE_F32, true);
+  const bool odd = vocab % 8 != 0;
+  auto launch = [&](auto dt, auto v, auto o) {
+    constexpr int DT = decltype(dt)::value;
+    constexpr bool V = decltype(v)::value, ODD = decltype(o)::value;
+    if (rows < kKlFewRows)
+      kl_rows_kernel<DT, V, ODD, 1024><<<grid, 1024, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_kl, row_nan);
     else
-      SF_KL_ROWS(SF_DTYPE_F32, false);
-  } else {
-    if (vec)
-      SF_KL_ROWS(SF_DTYPE_BF16, true);
-    else
-      SF_KL_ROWS(SF_DTYPE_BF16, false);
-  }
-#undef SF_KL_ROWS
+      kl_rows_kernel<DT, V, ODD, 256><<<grid, 256, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_kl, row_nan);
+  };
+  kl_dispatch(dtype, vec, odd, launch);
   const float t_sq = static_cast<float>(static_cast<double>(temperature) * static_cast<double>(temperature));
   kl_final_kernel<<<1, kKlFinalBlock, 0, st>>>(row_kl, row_nan, rows, chunk_rows, temperature, t_sq, row_scale, out,
                                                out_dtype);
@@ -478,26 +492,17 @@ extern "C" int sf_kl_backward(const void* student, const void* teacher, int dtyp
   const bool vec = kl_vec_ok({student, teacher, grad_student});
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 grid(static_cast<unsigned>(rows));
-#define SF_KL_BWD(DT, V)                                                                                          \
-  do {                                                                                                            \
-    if (rows < kKlFewRows)                                                                                        \
-      kl_backward_kernel<DT, V, 1024><<<grid, 1024, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_scale,  \
-                                                             grad_out, grad_out_dtype, grad_student);             \
-    else                                                                                                          \
-      kl_backward_kernel<DT, V, 256><<<grid, 256, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_scale,    \
-                                                           grad_out, grad_out_dtype, grad_student);               \
-  } while (0)
-  if (dtype == SF_DTYPE_F32) {
-    if (vec)
-      SF_KL_BWD(SF_DTYPE_F32, true);
+  const bool odd = vocab % 8 != 0;
+  auto launch = [&](auto dt, auto v, auto o) {
+    constexpr int DT = decltype(dt)::value;
+    constexpr bool V = decltype(v)::value, ODD = decltype(o)::value;
+    if (rows < kKlFewRows)
+      kl_backward_kernel<DT, V, ODD, 1024><<<grid, 1024, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_scale,
+                                                                  grad_out, grad_out_dtype, grad_student);
     else
-      SF_KL_BWD(SF_DTYPE_F32, false);
-  } else {
-    if (vec)
-      SF_KL_BWD(SF_DTYPE_BF16, true);
-    else
-      SF_KL_BWD(SF_DTYPE_BF16, false);
-  }
-#undef SF_KL_BWD
+      kl_backward_kernel<DT, V, ODD, 256><<<grid, 256, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_scale,
+                                                                grad_out, grad_out_dtype, grad_student);
+  };
+  kl_dispatch(dtype, vec, odd, launch);
   return launch_status("sf_kl_backward");
 }
