@@ -476,6 +476,18 @@ def _fused_attention_takes(q, k, v, cos, sin) -> bool:
             and all(not t.is_contiguous() or t.data_ptr() % 16 == 0 for t in (q, k, v, cos, sin)))
 
 
+def _attention_grads_by_passes(q, k, v, cos, sin, go, needed):
+    """Gradients of the materialised path (differentiable under create_graph) with respect to q, k, v where needed.
+    They are taken at views of the inputs: with respect to q, k, v themselves each would be the derivative through the
+    other two as well where those share a tensor or depend on each other, and would run the inputs' hooks once more."""
+    create_graph = torch.is_grad_enabled()
+    with torch.enable_grad():
+        views = [t.view_as(t) for t in (q, k, v)]
+        o = _causal_attention_device(*views, cos, sin)
+    grads = iter(torch.autograd.grad(o, [t for t, n in zip(views, needed) if n], go, create_graph=create_graph))
+    return [next(grads) if n else None for n in needed]
+
+
 class _FusedAttention(torch.autograd.Function):
     """causal_attention of bf16 heads with the S x S products kept in registers (sf_attention_forward /
     sf_attention_backward).  When the gradient itself is differentiated (create_graph, the Hutchinson probe)
@@ -499,12 +511,7 @@ class _FusedAttention(torch.autograd.Function):
     def backward(ctx, go):
         q, k, v, cos, sin, qr, kr, out, lse = ctx.saved_tensors
         if not plain_backward():  # create_graph, or a transform that the passes' own Functions take or refuse
-            wanted = [t for t, n in zip((q, k, v), ctx.needs_input_grad) if n]
-            create_graph = torch.is_grad_enabled()
-            with torch.enable_grad():
-                o = _causal_attention_device(q, k, v, cos, sin)
-            grads = iter(torch.autograd.grad(o, wanted, go, create_graph=create_graph))
-            return (*(next(grads) if n else None for n in ctx.needs_input_grad[:3]), None, None)
+            return (*_attention_grads_by_passes(q, k, v, cos, sin, go, ctx.needs_input_grad[:3]), None, None)
         dev = q.device
         B, S, H, D = q.shape
         go = _aligned(go.to(q.dtype))
