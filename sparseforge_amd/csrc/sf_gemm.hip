@@ -485,18 +485,27 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, const f32x16_t 
           ep[r * kEpiPitch + j * 32 + (lane & 31)] = acc[(2 * h + ii) * kFragN + j][e];
         }
     __syncthreads();
-    for (int it = 0; it < 16; ++it) {
-      const int flat = it * 64 + lane;
-      const int r = flat >> 4, c = (flat & 15) * 8;
-      const int64_t row = wrow0 + h * 64 + r, col = wcol0 + c;
-      if (row >= g.M || col >= g.N) continue;
-      float v[8];
-      const float4 p0 = *reinterpret_cast<const float4*>(ep + r * kEpiPitch + c);
-      const float4 p1 = *reinterpret_cast<const float4*>(ep + r * kEpiPitch + c + 4);
-      v[0] = p0.x; v[1] = p0.y; v[2] = p0.z; v[3] = p0.w;
-      v[4] = p1.x; v[5] = p1.y; v[6] = p1.z; v[7] = p1.w;
-      store_c8<Tr<T>::DT>(g, row, col, kz, v);
-    }
+    // Two loops, so that the one of products without a mask has no mask code: with both in one, every product's
+    // epilogue took about 1.4 us more per round of 256 tiles (8192, 8192, 64 63 us against 57; 8192, 8192, 1024 154
+    // against 148; with a bias 147 and 140).
+    auto rows = [&](auto masked) {
+      for (int it = 0; it < 16; ++it) {
+        const int flat = it * 64 + lane;
+        const int r = flat >> 4, c = (flat & 15) * 8;
+        const int64_t row = wrow0 + h * 64 + r, col = wcol0 + c;
+        if (row >= g.M || col >= g.N) continue;
+        float v[8];
+        const float4 p0 = *reinterpret_cast<const float4*>(ep + r * kEpiPitch + c);
+        const float4 p1 = *reinterpret_cast<const float4*>(ep + r * kEpiPitch + c + 4);
+        v[0] = p0.x; v[1] = p0.y; v[2] = p0.z; v[3] = p0.w;
+        v[4] = p1.x; v[5] = p1.y; v[6] = p1.z; v[7] = p1.w;
+        store_c8<Tr<T>::DT, decltype(masked)::value>(g, row, col, kz, v);
+      }
+    };
+    if (g.emask)
+      rows(std::true_type{});
+    else
+      rows(std::false_type{});
   }
 }
 

@@ -126,8 +126,8 @@ struct GemmArgs {
 namespace {
 // 8 consecutive columns of one row of a product (its f32 sums v): to the K split's partials, to the kept blocks of a
 // block-sparse C, or through the epilogue (output rounding, bias, mask product / decay term, accumulation) to C.
-// EDT: dtype of emask and dw.
-template <int EDT>
+// EDT: dtype of emask and dw; MASKED = false: there is no emask (a test outside the caller's loop).
+template <int EDT, bool MASKED = true>
 __device__ __forceinline__ void store_c8(const GemmArgs& g, int64_t row, int64_t col, int64_t kz, float (&v)[8]) {
   const bool cbf = g.c_dtype == SF_DTYPE_BF16;
   if (g.c_blocks) {
@@ -161,8 +161,8 @@ __device__ __forceinline__ void store_c8(const GemmArgs& g, int64_t row, int64_t
   }
   const int64_t off = row * g.ldc + col;
   const bool vec = g.c_aligned && col + 8 <= g.N && (off & 7) == 0 &&
-                   (!g.emask || (reinterpret_cast<uintptr_t>(g.emask) & 15u) == 0);
-  if (!g.dw && vec) {
+                   (!MASKED || !g.emask || (reinterpret_cast<uintptr_t>(g.emask) & 15u) == 0);
+  if ((!MASKED || !g.dw) && vec) {
     // result of the matmul in the output dtype, then + bias (rounded again), then + C when
     // accumulating: the per-element sequence below, 8 outputs at a time
     if (g.bias) {
@@ -172,7 +172,7 @@ __device__ __forceinline__ void store_c8(const GemmArgs& g, int64_t row, int64_t
         v[q] = cbf ? hround(v[q]) + b : v[q] + b;
       }
     }
-    if (g.emask) {  // times the effective mask, after the product (+ bias) is rounded
+    if (MASKED && g.emask) {  // times the effective mask, after the product (+ bias) is rounded
       float em[8];
       if constexpr (EDT == SF_DTYPE_BF16) {
         const uint4 ew = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(g.emask) + off);
@@ -225,7 +225,7 @@ __device__ __forceinline__ void store_c8(const GemmArgs& g, int64_t row, int64_t
       const float b = load_elem(g.bias, col + q, g.bias_dtype);
       x = cbf ? hround(x + b) : x + b;
     }
-    if (g.emask) {
+    if (MASKED && g.emask) {
       const float em = load_elem(g.emask, o, edt);
       if (g.dw) {
         if (em < 0.5f) {

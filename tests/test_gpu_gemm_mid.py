@@ -31,7 +31,8 @@ def test_layouts(cuda_device, M, N, K, layout):
         assert gemm_err(getattr(lin, "mm_" + layout)(A, B, max_splits=cap), ref, torch.bfloat16) <= 1.0
 
 
-@pytest.mark.parametrize("M,N,K,R", [(80, 96, 128, 8), (1000, 264, 520, 72), (200, 2048, 4096, 64)])
+@pytest.mark.parametrize("M,N,K,R", [(80, 96, 128, 8), (1000, 264, 520, 72), (200, 2048, 4096, 64),
+                                     (5632, 2048, 1032, 64)])  # the last on 256 x 256 tiles
 def test_segment_bias_mask_accumulate(cuda_device, M, N, K, R):
     from sparseforge_amd import linear as lin
 
