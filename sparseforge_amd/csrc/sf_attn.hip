@@ -249,8 +249,10 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnArgs a, int nb) {
   f32x16_t o[D / 32];
 #pragma unroll
   for (int i = 0; i < D / 32; ++i) o[i] = f32x16_t{};
-  float m = -INFINITY, l = 0.0f;  // of this lane's query; l over the keys this half-wave holds
   const float c = a.scale * kLog2e;
+  // of this lane's query: the largest score so far times c, what is subtracted for it (0 while every score is -inf, so
+  // that those count 0 and not NaN), and the sum over the keys this half-wave holds
+  float m = -INFINITY, ms = 0.0f, l = 0.0f;
   const int64_t end = (int64_t)(blk + 1) * kAtRows < a.S ? (int64_t)(blk + 1) * kAtRows : a.S;
   const int nt = static_cast<int>(ceil_div(end, kAtTile));
   AtTile<D> tk, tv;
@@ -290,19 +292,20 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnArgs a, int nb) {
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * c;
     const float mn = fmaxf(m, mx);
     if (__builtin_amdgcn_ballot_w64(mn > m) != 0) {  // some query's maximum rose: rescale what is accumulated
-      const float al = __builtin_amdgcn_exp2f(m - mn);
+      const float mns = mn == -INFINITY ? 0.0f : mn, al = __builtin_amdgcn_exp2f(m - mns);
       l *= al;
 #pragma unroll
       for (int i = 0; i < D / 32; ++i)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[i][e] *= al;
       m = mn;
+      ms = mns;
     }
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        s[b][e] = __builtin_amdgcn_exp2f(fmaf(s[b][e], c, -m));
+        s[b][e] = __builtin_amdgcn_exp2f(fmaf(s[b][e], c, -ms));
         l += s[b][e];
       }
 #pragma unroll

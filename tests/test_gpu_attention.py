@@ -96,3 +96,28 @@ def test_calls_outside_the_fused_path(cuda_device):
         assert not llama._fused_attention_takes(q, k, v, cos, sin)
         assert torch.equal(llama.causal_attention(q, k, v, cos, sin),
                            llama._causal_attention_device(q, k, v, cos, sin))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_first_keys_at_minus_infinity(cuda_device, D):
+    """Queries whose first tile of 64 keys (and 6 more) scores -inf in float32, the rest finite: those keys get
+    probability 0 and nothing becomes NaN."""
+    from sparseforge_amd import llama
+
+    S = 200
+    q, k, v, go = (torch.randn(1, S, 2, D, device=cuda_device) for _ in range(4))
+    q[:, :70], q[:, 70:] = 1e-19, 1e18     # 1e18 * -1e21 * D overflows; 1e-19 * -1e21 * D does not
+    k[:, :70] = -1e21
+    k[:, 70:] *= 1e-18
+    go[:, :70] = 0                         # those queries' dq is a cancelling sum of terms of 1e21
+    q, k, v, go = (t.to(torch.bfloat16) for t in (q, k, v, go.reshape(1, S, 2 * D)))
+    q, k, v = (t.requires_grad_(True) for t in (q, k, v))
+    cos, sin = torch.ones(S, D, device=cuda_device), torch.zeros(S, D, device=cuda_device)  # no rotation
+    o = llama.causal_attention(q, k, v, cos, sin)
+    grads = torch.autograd.grad(o, (q, k, v), go)
+    ro, rg = _ref(q, k, v, cos, sin, go)
+    for part in (slice(0, 70), slice(70, S)):  # gradients of the two parts differ by orders of magnitude
+        for got, want in zip((o, *grads), (ro, *rg)):
+            a, b = got.detach()[:, part].double(), want.detach()[:, part].double()
+            assert torch.isfinite(a).all()
+            assert float((a - b).norm()) <= 1e-2 * float(b.norm()) + 1e-30 * a.numel()
