@@ -3,10 +3,16 @@
 // retrains with, legacy/model_llama.py:39-55; the Hutchinson double backward
 // keeps the materialised products of llama._causal_attention_device).
 //
-//   forward   o = softmax(scale q k^T, causal) v, and per row the base-2 log of
-//             the softmax's denominator (max included)
-//   backward  p = exp2(scale log2e s - lse),  ds = p (do v^T - delta),
+//   forward   o = softmax(scale q k^T, causal) v, and per row its largest score and
+//             the base-2 log of the sum of 2^(c (score - largest)), c = scale log2e
+//   backward  p = exp2(c s - lse), lse = c largest + log,  ds = p (do v^T - delta),
 //             delta = sum_d do o;  dv = p^T do, dk = scale ds^T q, dq = scale ds k
+//
+// c s - lse as one fused multiply-add leaves what rounding lse to f32 loses, 2^-13
+// at kAtBig; beyond that (scores that have run away) the maximum is subtracted from
+// the score first, which is exact at any size but costs another instruction per
+// element.  The forward and dq decide that per wave; dk / dv, where a test per tile
+// cost 11 of 147 us, by one word that the forward sets, with a body for each case.
 //
 // The scores, the probabilities' sums and every accumulation stay f32 in
 // registers; p and ds round to bf16 as operands of the next product, as the
@@ -41,6 +47,7 @@ namespace {
 
 constexpr int kAtRows = 128;  // queries (forward, dq) or keys (dk / dv) of a workgroup: 4 waves of 32
 constexpr int kAtTile = 64;   // the other side's tile
+constexpr float kAtBig = 4096.0f;  // |c score| from which the row's maximum is subtracted before c is applied
 typedef short v4i16_t __attribute__((ext_vector_type(4)));
 
 struct AttnArgs {
@@ -49,7 +56,7 @@ struct AttnArgs {
   const uint16_t* v;
   const uint16_t* go;  // gradient of the output (backward)
   const uint16_t* o;
-  float* lse;          // [B H, S]
+  float* stats;        // [3][B H, S]: lse, largest score, log2 of the sum; then one word, not 0 if a score is past kAtBig
   float* delta;        // [B H, S]
   uint16_t* out;       // forward: o
   uint16_t* dq;
@@ -66,6 +73,8 @@ struct AttnArgs {
 // banks and the transposed reads of 4 rows x 64 bytes overlap in 4 words only.
 template <int D>
 constexpr int at_pitch() { return D == 64 ? 208 : 336; }
+
+__host__ __device__ __forceinline__ float* at_flag(const AttnArgs& a) { return a.stats + 3 * (int64_t)a.BH * a.S; }
 
 // Block order: the row blocks of one (batch, head) on one XCD, `last` first when its rows are the longest.
 __device__ __forceinline__ void at_block(const AttnArgs& a, int nb, bool last_first, int& bh, int& blk) {
@@ -163,7 +172,8 @@ template <int D>
 __global__ void __launch_bounds__(256) rotate_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
                                                      uint16_t* __restrict__ qr, uint16_t* __restrict__ kr,
                                                      const float* __restrict__ cos, const float* __restrict__ sin,
-                                                     int64_t S, int H, int64_t work) {
+                                                     int64_t S, int H, int64_t work, float* __restrict__ flag) {
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *flag = 0.0f;  // the forward kernel may set it
   constexpr int C = D / 16;  // chunks of 8 in half a head
   const int64_t i = blockIdx.x * 256ll + threadIdx.x;
   if (i >= work) return;
@@ -250,9 +260,11 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnArgs a, int nb) {
 #pragma unroll
   for (int i = 0; i < D / 32; ++i) o[i] = f32x16_t{};
   const float c = a.scale * kLog2e;
-  // of this lane's query: the largest score so far times c, what is subtracted for it (0 while every score is -inf, so
-  // that those count 0 and not NaN), and the sum over the keys this half-wave holds
-  float m = -INFINITY, ms = 0.0f, l = 0.0f;
+  // of this lane's query: the largest score so far, that score (0 while every score is -inf, so that those count 0 and
+  // not NaN) and it times c, and the sum over the keys this half-wave holds
+  float m = -INFINITY, mz = 0.0f, ms = 0.0f, l = 0.0f;
+  float sub = 0.0f;  // ms, or 0 if big
+  bool big = false;  // some query of the wave: |ms| > kAtBig; then mz is taken from the scores as they come
   const int64_t end = (int64_t)(blk + 1) * kAtRows < a.S ? (int64_t)(blk + 1) * kAtRows : a.S;
   const int nt = static_cast<int>(ceil_div(end, kAtTile));
   AtTile<D> tk, tv;
@@ -289,23 +301,34 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnArgs a, int nb) {
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[b][e]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * c;
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     const float mn = fmaxf(m, mx);
-    if (__builtin_amdgcn_ballot_w64(mn > m) != 0) {  // some query's maximum rose: rescale what is accumulated
-      const float mns = mn == -INFINITY ? 0.0f : mn, al = __builtin_amdgcn_exp2f(m - mns);
+    if (big || __builtin_amdgcn_ballot_w64(mn > m) != 0) {  // some query's maximum rose: rescale what is accumulated
+      const float nz = mn == -INFINITY ? 0.0f : mn, ns = nz * c;
+      big = __builtin_amdgcn_ballot_w64(fabsf(ns) > kAtBig) != 0;
+      const float al = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(big ? (mz - nz) * c : ms - ns);
       l *= al;
 #pragma unroll
       for (int i = 0; i < D / 32; ++i)
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[i][e] *= al;
       m = mn;
-      ms = mns;
+      mz = nz;
+      ms = ns;
+      sub = ms;
+      if (big) {
+        sub = 0.0f;
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) s[b][e] -= mz;
+      }
     }
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        s[b][e] = __builtin_amdgcn_exp2f(fmaf(s[b][e], c, -ms));
+        s[b][e] = __builtin_amdgcn_exp2f(fmaf(s[b][e], c, -sub));
         l += s[b][e];
       }
 #pragma unroll
@@ -320,7 +343,14 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnArgs a, int nb) {
   }
   l += __shfl_xor(l, 32, 64);
   store_rows<D, false>(a.out, a, bh, q0, o, 1.0f / l);
-  if (lane < 32 && query < a.S) a.lse[bh * a.S + query] = m + __builtin_amdgcn_logf(l);
+  if (lane < 32 && query < a.S) {
+    const float lg = __builtin_amdgcn_logf(l), lse = m * c + lg;
+    float* st = a.stats + bh * a.S + query;
+    st[0] = lse;
+    st[a.BH * a.S] = m;
+    st[2 * a.BH * a.S] = lg;
+    if (fabsf(lse) > kAtBig) *at_flag(a) = 1.0f;  // the same value from every such query
+  }
 }
 
 // delta[bh, s] = sum_d go o: one thread per 8 dims, folded over the row's D / 8 threads.
@@ -359,12 +389,18 @@ __global__ void __launch_bounds__(256, 2) attn_dq_kernel(AttnArgs a, int nb) {
   bf16x8_t qf[D / 16], gf[D / 16];
   own_frags<D>(at_rows<D>(a.q, a, bh), q0, a.H, qf);
   own_frags<D>(at_rows<D>(a.go, a, bh), q0, a.H, gf);
-  const float lse = query < a.S ? a.lse[bh * a.S + query] : INFINITY;
+  const float c = a.scale * kLog2e;
+  const float* st = a.stats + bh * a.S + query;
+  float sub = query < a.S ? st[0] : INFINITY, mz = 0.0f;
+  const bool big = __builtin_amdgcn_ballot_w64(query < a.S && fabsf(sub) > kAtBig) != 0;
+  if (big && query < a.S) {
+    mz = st[a.BH * a.S];
+    sub = st[2 * a.BH * a.S];
+  }
   const float delta = query < a.S ? a.delta[bh * a.S + query] : 0.0f;
   f32x16_t dq[D / 32];
 #pragma unroll
   for (int i = 0; i < D / 32; ++i) dq[i] = f32x16_t{};
-  const float c = a.scale * kLog2e;
   const int64_t end = (int64_t)(blk + 1) * kAtRows < a.S ? (int64_t)(blk + 1) * kAtRows : a.S;
   const int nt = static_cast<int>(ceil_div(end, kAtTile));
   AtTile<D> tk, tv;
@@ -390,9 +426,13 @@ __global__ void __launch_bounds__(256, 2) attn_dq_kernel(AttnArgs a, int nb) {
         s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(kb, b * 32, kk), qf[kk], s, 0, 0, 0);
         dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(vb, b * 32, kk), gf[kk], dp, 0, 0, 0);
       }
+      if (__builtin_expect(big, 0)) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[e] -= mz;
+      }
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        float p = __builtin_amdgcn_exp2f(fmaf(s[e], c, -lse));
+        float p = __builtin_amdgcn_exp2f(fmaf(s[e], c, -sub));
         if (diag && n0 + b * 32 + acc_row(e) > query) p = 0.0f;
         s[e] = p * (dp[e] - delta);
       }
@@ -412,10 +452,13 @@ __global__ void __launch_bounds__(256, 2) attn_dq_kernel(AttnArgs a, int nb) {
 // dk, dv: 128 keys of one (batch, head), tiles of 64 queries from the diagonal on.
 // ---------------------------------------------------------------------------
 template <int D>
-__global__ void __launch_bounds__(256, D == 64 ? 2 : 1) attn_dkv_kernel(AttnArgs a, int nb) {
-  __shared__ __align__(16) unsigned char qs[2][kAtTile * at_pitch<D>()];
-  __shared__ __align__(16) unsigned char gs[2][kAtTile * at_pitch<D>()];
-  __shared__ __align__(16) float rows_s[2][2][kAtTile];  // lse, delta of the tile's queries
+struct DkvLds {
+  unsigned char q[2][kAtTile * at_pitch<D>()];
+  unsigned char g[2][kAtTile * at_pitch<D>()];
+  float rows[2][3][kAtTile];  // of the tile's queries: lse (BIG: log2 of the sum), delta, maximum
+};
+template <int D, bool BIG>
+__device__ __forceinline__ void attn_dkv_block(const AttnArgs& a, int nb, DkvLds<D>& sm) {
   int bh, blk;
   at_block(a, nb, false, bh, blk);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h4 = (lane >> 5) * 4;
@@ -430,23 +473,28 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) attn_dkv_kernel(AttnArgs
   const float c = a.scale * kLog2e;
   const int t0 = blk * (kAtRows / kAtTile), nt = static_cast<int>(ceil_div(a.S, kAtTile));
   AtTile<D> tq, tg;
-  float row_v = 0.0f;  // threads 0..63: lse of the next tile's query, 64..127: its delta
+  // threads 0..63: lse of the next tile's query (BIG: log2 of its sum, and its maximum), 64..127: its delta
+  float row_v = 0.0f, row_m = 0.0f;
   auto load_rows = [&](int t) {
     const int64_t s = (int64_t)t * kAtTile + (threadIdx.x & 63);
-    if (threadIdx.x < 64)
-      row_v = s < a.S ? a.lse[bh * a.S + s] : INFINITY;  // past the end: p = 0
-    else if (threadIdx.x < 128)
+    if (threadIdx.x < 64) {
+      row_v = s < a.S ? a.stats[((BIG ? 2 * a.BH : 0) + bh) * a.S + s] : INFINITY;  // past the end: p = 0
+      if constexpr (BIG) row_m = s < a.S ? a.stats[(a.BH + bh) * a.S + s] : 0.0f;
+    } else if (threadIdx.x < 128) {
       row_v = s < a.S ? a.delta[bh * a.S + s] : 0.0f;
+    }
   };
   tq.load(rq, (int64_t)t0 * kAtTile, a.H);
   tg.load(rg, (int64_t)t0 * kAtTile, a.H);
   load_rows(t0);
   for (int t = t0; t < nt; ++t) {
     const int buf = (t - t0) & 1;
-    unsigned char *qb = qs[buf], *gb = gs[buf];
+    unsigned char *qb = sm.q[buf], *gb = sm.g[buf];
     tq.store(qb);
     tg.store(gb);
-    if (threadIdx.x < 128) rows_s[buf][threadIdx.x >> 6][threadIdx.x & 63] = row_v;
+    if (threadIdx.x < 128) sm.rows[buf][threadIdx.x >> 6][threadIdx.x & 63] = row_v;
+    if constexpr (BIG)
+      if (threadIdx.x < 64) sm.rows[buf][2][threadIdx.x] = row_m;
     __syncthreads();
     const int64_t n0 = (int64_t)t * kAtTile;
     if (t + 1 < nt) {
@@ -464,11 +512,20 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) attn_dkv_kernel(AttnArgs
         s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(qb, b * 32, kk), kf[kk], s, 0, 0, 0);
         dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(row_frag<D>(gb, b * 32, kk), vf[kk], dp, 0, 0, 0);
       }
+      if constexpr (BIG) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float4 mx = *reinterpret_cast<const float4*>(&sm.rows[buf][2][b * 32 + g * 8 + h4]);
+          const float m4[4] = {mx.x, mx.y, mx.z, mx.w};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) s[4 * g + j] -= m4[j];
+        }
+      }
       f32x16_t p;
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const float4 ls = *reinterpret_cast<const float4*>(&rows_s[buf][0][b * 32 + g * 8 + h4]);
-        const float4 de = *reinterpret_cast<const float4*>(&rows_s[buf][1][b * 32 + g * 8 + h4]);
+        const float4 ls = *reinterpret_cast<const float4*>(&sm.rows[buf][0][b * 32 + g * 8 + h4]);
+        const float4 de = *reinterpret_cast<const float4*>(&sm.rows[buf][1][b * 32 + g * 8 + h4]);
         const float l4[4] = {ls.x, ls.y, ls.z, ls.w}, d4[4] = {de.x, de.y, de.z, de.w};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -493,6 +550,15 @@ __global__ void __launch_bounds__(256, D == 64 ? 2 : 1) attn_dkv_kernel(AttnArgs
   store_rows<D, true>(a.dk, a, bh, k0, dk, a.scale);
 }
 
+template <int D>
+__global__ void __launch_bounds__(256, D == 64 ? 2 : 1) attn_dkv_kernel(AttnArgs a, int nb) {
+  __shared__ __align__(16) DkvLds<D> sm;
+  if (__builtin_expect(*at_flag(a) != 0.0f, 0))
+    attn_dkv_block<D, true>(a, nb, sm);
+  else
+    attn_dkv_block<D, false>(a, nb, sm);
+}
+
 bool at_ok(int64_t B, int64_t S, int64_t H, int64_t D) {
   return B > 0 && S > 0 && H > 0 && (D == 64 || D == 128) && S * H * D * 2 < (int64_t(1) << 31) &&
          B * H * ceil_div(S, kAtRows) < (int64_t(1) << 31) && B * S * H * (D / 8) < (int64_t(1) << 31);
@@ -504,7 +570,7 @@ int attn_forward(AttnArgs a, const uint16_t* q, const uint16_t* k, uint16_t* qr,
                  hipStream_t st) {
   const int64_t work = B * a.S * a.H * (D / 16);
   rotate_kernel<D><<<dim3(static_cast<unsigned>(ceil_div(work, 256)), 2), 256, 0, st>>>(q, k, qr, kr, a.cos, a.sin, a.S,
-                                                                                       a.H, work);
+                                                                                       a.H, work, at_flag(a));
   const int nb = static_cast<int>(ceil_div(a.S, kAtRows));
   attn_fwd_kernel<D><<<a.BH * nb, 256, 0, st>>>(a, nb);
   return launch_status("sf_attention_forward");
@@ -525,19 +591,19 @@ int attn_backward(AttnArgs a, int64_t B, hipStream_t st) {
 using namespace sf;
 
 extern "C" int sf_attention_forward(const void* q, const void* k, const void* v, int64_t B, int64_t S, int64_t H,
-                                    int64_t D, const float* cos, const float* sin, float scale, void* out, float* lse,
+                                    int64_t D, const float* cos, const float* sin, float scale, void* out, float* row_stats,
                                     void* q_rot, void* k_rot, void* stream) {
   SF_CHECK_ARG(at_ok(B, S, H, D), "attention: unsupported shape B=%lld S=%lld H=%lld D=%lld", (long long)B,
                (long long)S, (long long)H, (long long)D);
   SF_CHECK_ARG(at_al(q) && at_al(k) && at_al(v) && at_al(out) && at_al(q_rot) && at_al(k_rot) && at_al(cos) &&
-                   at_al(sin) && lse,
+                   at_al(sin) && row_stats,
                "attention: null or unaligned tensor");
   AttnArgs a = {};
   a.q = static_cast<const uint16_t*>(q_rot);
   a.k = static_cast<const uint16_t*>(k_rot);
   a.v = static_cast<const uint16_t*>(v);
   a.out = static_cast<uint16_t*>(out);
-  a.lse = lse;
+  a.stats = row_stats;
   a.cos = cos;
   a.sin = sin;
   a.S = S;
@@ -551,13 +617,13 @@ extern "C" int sf_attention_forward(const void* q, const void* k, const void* v,
 }
 
 extern "C" int sf_attention_backward(const void* q_rot, const void* k_rot, const void* v, const void* out,
-                                     const void* grad_out, const float* lse, int64_t B, int64_t S, int64_t H,
+                                     const void* grad_out, const float* row_stats, int64_t B, int64_t S, int64_t H,
                                      int64_t D, const float* cos, const float* sin, float scale, float* delta,
                                      void* dq, void* dk, void* dv, void* stream) {
   SF_CHECK_ARG(at_ok(B, S, H, D), "attention: unsupported shape B=%lld S=%lld H=%lld D=%lld", (long long)B,
                (long long)S, (long long)H, (long long)D);
   SF_CHECK_ARG(at_al(q_rot) && at_al(k_rot) && at_al(v) && at_al(out) && at_al(grad_out) && at_al(dq) && at_al(dk) &&
-                   at_al(dv) && at_al(cos) && at_al(sin) && lse && delta,
+                   at_al(dv) && at_al(cos) && at_al(sin) && row_stats && delta,
                "attention: null or unaligned tensor");
   AttnArgs a = {};
   a.q = static_cast<const uint16_t*>(q_rot);
@@ -565,7 +631,7 @@ extern "C" int sf_attention_backward(const void* q_rot, const void* k_rot, const
   a.v = static_cast<const uint16_t*>(v);
   a.o = static_cast<const uint16_t*>(out);
   a.go = static_cast<const uint16_t*>(grad_out);
-  a.lse = const_cast<float*>(lse);
+  a.stats = const_cast<float*>(row_stats);
   a.delta = delta;
   a.dq = static_cast<uint16_t*>(dq);
   a.dk = static_cast<uint16_t*>(dk);

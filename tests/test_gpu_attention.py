@@ -121,3 +121,30 @@ def test_first_keys_at_minus_infinity(cuda_device, D):
             a, b = got.detach()[:, part].double(), want.detach()[:, part].double()
             assert torch.isfinite(a).all()
             assert float((a - b).norm()) <= 1e-2 * float(b.norm()) + 1e-30 * a.numel()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("size", [1.0, 30.0, 1e3, 1e6, 1e15])
+def test_runaway_scores(cuda_device, D, size):
+    """Scores up to 2^100 (one key takes all, or the first two share: they are equal) in all heads but the first, forward
+    and backward.  dq, which cancels exactly where two equal keys share, only has to be finite."""
+    from sparseforge_amd import llama
+
+    S = 150
+    g = torch.Generator(device=cuda_device).manual_seed(D)
+    q, k, v, go = (torch.randn(1, S, 4, D, generator=g, device=cuda_device) for _ in range(4))
+    k[:, :2] = 3 * k[:, :1]  # the first two keys take many rows
+    q[:, :, 1:] *= size
+    k[:, :, 1:] *= size
+    q, k, v, go = (t.to(torch.bfloat16) for t in (q, k, v, go.reshape(1, S, 4 * D)))
+    q, k, v = (t.requires_grad_(True) for t in (q, k, v))
+    cos, sin = torch.ones(S, D, device=cuda_device), torch.zeros(S, D, device=cuda_device)  # no rotation
+    o = llama.causal_attention(q, k, v, cos, sin)
+    grads = torch.autograd.grad(o, (q, k, v), go)
+    ro, rg = _ref(q, k, v, cos, sin, go)
+    assert torch.isfinite(grads[0]).all()
+    for got, want in ((o, ro), (grads[1], rg[1]), (grads[2], rg[2])):
+        got, want = (t.detach().double().view(S, 4, D) for t in (got, want))
+        assert torch.isfinite(got).all()
+        for h in range(4):
+            assert float((got[:, h] - want[:, h]).norm() / want[:, h].norm()) < 1e-2
