@@ -568,7 +568,8 @@ int sf_from_heads(const void* g, int dtype, int64_t B, int64_t S, int64_t H, int
  * tensor below 2 GiB per batch entry and 16-byte aligned.
  *   forward:  q_rot, k_rot = rot(q), rot(k) (sf_to_heads' rotation, kept for the
  *             backward), out = softmax(scale q_rot k_rot^T, causal) v with the
- *             scores and sums in f32; row_stats [3 B H S + 1] = per row the base-2
+ *             scores and sums in f32; out_f32 = out before its rounding, for the
+ *             backward (may be null without one); row_stats [3 B H S + 1] = per row the base-2
  *             logarithm of its sum of 2^(scale log2(e) score), its largest score
  *             (unscaled) and the logarithm of its sum of 2^(scale log2(e) (score -
  *             largest)), then a word that is not 0 where a score is so large that
@@ -577,10 +578,10 @@ int sf_from_heads(const void* g, int dtype, int64_t B, int64_t S, int64_t H, int
  *             delta [B * H, S] f32 is scratch
  */
 int sf_attention_forward(const void* q, const void* k, const void* v, int64_t B, int64_t S, int64_t H, int64_t D,
-                         const float* cos, const float* sin, float scale, void* out, float* row_stats, void* q_rot,
-                         void* k_rot, void* stream);
-int sf_attention_backward(const void* q_rot, const void* k_rot, const void* v, const void* out, const void* grad_out,
-                          const float* row_stats, int64_t B, int64_t S, int64_t H, int64_t D, const float* cos,
+                         const float* cos, const float* sin, float scale, void* out, float* out_f32,
+                         float* row_stats, void* q_rot, void* k_rot, void* stream);
+int sf_attention_backward(const void* q_rot, const void* k_rot, const void* v, const float* out_f32,
+                          const void* grad_out, const float* row_stats, int64_t B, int64_t S, int64_t H, int64_t D, const float* cos,
                           const float* sin, float scale, float* delta, void* dq, void* dk, void* dv, void* stream);
 
 /*

@@ -55,7 +55,7 @@ struct AttnArgs {
   const uint16_t* k;   // rotated
   const uint16_t* v;
   const uint16_t* go;  // gradient of the output (backward)
-  const uint16_t* o;
+  float* o32;          // [B, S, H, D]: the output before it is rounded (forward: null without a backward)
   float* stats;        // [3][B H, S]: lse, largest score, log2 of the sum; then one word, not 0 if a score is past kAtBig
   float* delta;        // [B H, S]
   uint16_t* out;       // forward: o
@@ -242,6 +242,23 @@ __device__ __forceinline__ void store_rows(uint16_t* t, const AttnArgs& a, int b
   }
 }
 
+// The same rows in f32, without rotation.
+template <int D>
+__device__ __forceinline__ void store_rows_f32(float* t, const AttnArgs& a, int bh, int64_t row0,
+                                               const f32x16_t (&acc)[D / 32], float f) {
+  const int lane = threadIdx.x & 63, h4 = (lane >> 5) * 4;
+  const int64_t row = row0 + (lane & 31);
+  if (row >= a.S) return;
+  const int64_t b = bh / a.H, h = bh - b * a.H;
+  float* dst = t + ((b * a.S + row) * a.H + h) * D;
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<float4*>(dst + db * 32 + g * 8 + h4) =
+          make_float4(acc[db][4 * g] * f, acc[db][4 * g + 1] * f, acc[db][4 * g + 2] * f, acc[db][4 * g + 3] * f);
+}
+
 // ---------------------------------------------------------------------------
 // Forward: 128 queries of one (batch, head).
 // ---------------------------------------------------------------------------
@@ -343,6 +360,7 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnArgs a, int nb) {
   }
   l += __shfl_xor(l, 32, 64);
   store_rows<D, false>(a.out, a, bh, q0, o, 1.0f / l);
+  if (a.o32) store_rows_f32<D>(a.o32, a, bh, q0, o, 1.0f / l);
   if (lane < 32 && query < a.S) {
     const float lg = __builtin_amdgcn_logf(l), lse = m * c + lg;
     float* st = a.stats + bh * a.S + query;
@@ -353,16 +371,18 @@ __global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnArgs a, int nb) {
   }
 }
 
-// delta[bh, s] = sum_d go o: one thread per 8 dims, folded over the row's D / 8 threads.
+// delta[bh, s] = sum_d go o: one thread per 8 dims, folded over the row's D / 8 threads.  From the forward's own f32
+// output: the one that it returns is rounded, and may have been changed in place since.
 template <int D>
 __global__ void __launch_bounds__(256) attn_delta_kernel(AttnArgs a, int64_t work) {
   constexpr int C = D / 8;
   const int64_t i = blockIdx.x * 256ll + threadIdx.x;
   float d = 0.0f;
   if (i < work) {
-    float x[8], y[8];
+    float x[8];
     unpack8(*reinterpret_cast<const uint4*>(a.go + i * 8), x);
-    unpack8(*reinterpret_cast<const uint4*>(a.o + i * 8), y);
+    const float4 y0 = *reinterpret_cast<const float4*>(a.o32 + i * 8), y1 = *reinterpret_cast<const float4*>(a.o32 + i * 8 + 4);
+    const float y[8] = {y0.x, y0.y, y0.z, y0.w, y1.x, y1.y, y1.z, y1.w};
 #pragma unroll
     for (int j = 0; j < 8; ++j) d = fmaf(x[j], y[j], d);
   }
@@ -591,18 +611,19 @@ int attn_backward(AttnArgs a, int64_t B, hipStream_t st) {
 using namespace sf;
 
 extern "C" int sf_attention_forward(const void* q, const void* k, const void* v, int64_t B, int64_t S, int64_t H,
-                                    int64_t D, const float* cos, const float* sin, float scale, void* out, float* row_stats,
-                                    void* q_rot, void* k_rot, void* stream) {
+                                    int64_t D, const float* cos, const float* sin, float scale, void* out, float* out_f32,
+                                    float* row_stats, void* q_rot, void* k_rot, void* stream) {
   SF_CHECK_ARG(at_ok(B, S, H, D), "attention: unsupported shape B=%lld S=%lld H=%lld D=%lld", (long long)B,
                (long long)S, (long long)H, (long long)D);
   SF_CHECK_ARG(at_al(q) && at_al(k) && at_al(v) && at_al(out) && at_al(q_rot) && at_al(k_rot) && at_al(cos) &&
-                   at_al(sin) && row_stats,
+                   at_al(sin) && row_stats && (!out_f32 || at_al(out_f32)),
                "attention: null or unaligned tensor");
   AttnArgs a = {};
   a.q = static_cast<const uint16_t*>(q_rot);
   a.k = static_cast<const uint16_t*>(k_rot);
   a.v = static_cast<const uint16_t*>(v);
   a.out = static_cast<uint16_t*>(out);
+  a.o32 = out_f32;
   a.stats = row_stats;
   a.cos = cos;
   a.sin = sin;
@@ -616,20 +637,20 @@ extern "C" int sf_attention_forward(const void* q, const void* k, const void* v,
   return D == 64 ? attn_forward<64>(a, qi, ki, qo, ko, B, st) : attn_forward<128>(a, qi, ki, qo, ko, B, st);
 }
 
-extern "C" int sf_attention_backward(const void* q_rot, const void* k_rot, const void* v, const void* out,
+extern "C" int sf_attention_backward(const void* q_rot, const void* k_rot, const void* v, const float* out_f32,
                                      const void* grad_out, const float* row_stats, int64_t B, int64_t S, int64_t H,
                                      int64_t D, const float* cos, const float* sin, float scale, float* delta,
                                      void* dq, void* dk, void* dv, void* stream) {
   SF_CHECK_ARG(at_ok(B, S, H, D), "attention: unsupported shape B=%lld S=%lld H=%lld D=%lld", (long long)B,
                (long long)S, (long long)H, (long long)D);
-  SF_CHECK_ARG(at_al(q_rot) && at_al(k_rot) && at_al(v) && at_al(out) && at_al(grad_out) && at_al(dq) && at_al(dk) &&
+  SF_CHECK_ARG(at_al(q_rot) && at_al(k_rot) && at_al(v) && at_al(out_f32) && at_al(grad_out) && at_al(dq) && at_al(dk) &&
                    at_al(dv) && at_al(cos) && at_al(sin) && row_stats && delta,
                "attention: null or unaligned tensor");
   AttnArgs a = {};
   a.q = static_cast<const uint16_t*>(q_rot);
   a.k = static_cast<const uint16_t*>(k_rot);
   a.v = static_cast<const uint16_t*>(v);
-  a.o = static_cast<const uint16_t*>(out);
+  a.o32 = const_cast<float*>(out_f32);
   a.go = static_cast<const uint16_t*>(grad_out);
   a.stats = const_cast<float*>(row_stats);
   a.delta = delta;

@@ -498,18 +498,20 @@ class _FusedAttention(torch.autograd.Function):
         dev = L.require_device(q, k, v, cos, sin)
         B, S, H, D = q.shape
         out = torch.empty((B, S, H * D), dtype=q.dtype, device=dev)
+        # the backward reads the output as it was computed: in float32, in a buffer that no caller changes in place
+        out32 = torch.empty((B, S, H * D), dtype=torch.float32, device=dev) if any(ctx.needs_input_grad[:3]) else None
         stats = torch.empty(3 * B * H * S + 1, dtype=torch.float32, device=dev)
         qr, kr = torch.empty_like(q), torch.empty_like(k)
         with _prof.region("sf_attention_forward", 4 * q.numel() * q.element_size(), "B", dev):
             L.check(L.lib().sf_attention_forward(L.ptr(q), L.ptr(k), L.ptr(v), B, S, H, D, L.ptr(cos), L.ptr(sin),
-                                                 D ** -0.5, L.ptr(out), L.ptr(stats), L.ptr(qr), L.ptr(kr),
+                                                 D ** -0.5, L.ptr(out), L.ptr(out32), L.ptr(stats), L.ptr(qr), L.ptr(kr),
                                                  L.stream(dev)), "sf_attention_forward")
-        ctx.save_for_backward(q, k, v, cos, sin, qr, kr, out, stats)
+        ctx.save_for_backward(q, k, v, cos, sin, qr, kr, out32, stats)
         return out
 
     @staticmethod
     def backward(ctx, go):
-        q, k, v, cos, sin, qr, kr, out, stats = ctx.saved_tensors
+        q, k, v, cos, sin, qr, kr, out32, stats = ctx.saved_tensors
         if not plain_backward():  # create_graph, or a transform that the passes' own Functions take or refuse
             return (*_attention_grads_by_passes(q, k, v, cos, sin, go, ctx.needs_input_grad[:3]), None, None)
         dev = q.device
@@ -518,7 +520,7 @@ class _FusedAttention(torch.autograd.Function):
         delta = torch.empty(B * H * S, dtype=torch.float32, device=dev)
         dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
         with _prof.region("sf_attention_backward", 8 * q.numel() * q.element_size(), "B", dev):
-            L.check(L.lib().sf_attention_backward(L.ptr(qr), L.ptr(kr), L.ptr(v), L.ptr(out), L.ptr(go), L.ptr(stats),
+            L.check(L.lib().sf_attention_backward(L.ptr(qr), L.ptr(kr), L.ptr(v), L.ptr(out32), L.ptr(go), L.ptr(stats),
                                                   B, S, H, D, L.ptr(cos), L.ptr(sin), D ** -0.5, L.ptr(delta),
                                                   L.ptr(dq), L.ptr(dk), L.ptr(dv), L.stream(dev)),
                     "sf_attention_backward")

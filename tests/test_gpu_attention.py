@@ -148,3 +148,40 @@ def test_runaway_scores(cuda_device, D, size):
         assert torch.isfinite(got).all()
         for h in range(4):
             assert float((got[:, h] - want[:, h]).norm() / want[:, h].norm()) < 1e-2
+
+
+def test_output_changed_in_place(cuda_device):
+    """The output may be changed in place before the backward, which then sees the change as an op of its own."""
+    from sparseforge_amd import llama
+
+    S, H, D = 70, 3, 64
+    q, k, v = (torch.randn(1, S, H, D, device=cuda_device).to(torch.bfloat16).requires_grad_(True) for _ in range(3))
+    go = torch.randn(1, S, H * D, device=cuda_device).to(torch.bfloat16)
+    cos, sin = llama.rotary_tables(S, D, 10000.0, cuda_device)
+    want = torch.autograd.grad(llama.causal_attention(q, k, v, cos, sin), (q, k, v), go * 2)
+    o = llama.causal_attention(q, k, v, cos, sin)
+    o.mul_(2)
+    for a, b in zip(torch.autograd.grad(o, (q, k, v), go), want):
+        assert torch.equal(a, b)
+
+
+def test_delta_from_the_unrounded_output(cuda_device):
+    """delta = sum(go o) from the output before its rounding.  With values of 100 +- 1 the gradients are what is left of
+    go v after delta, about 8; the output's rounding (0.14 rms at 100) would move delta by 0.14 sqrt(64) = 1.15, 14 %.
+    The forward's own rounding of p moves o by 100 2^-9 / sqrt(3 n) over n keys, below 7e-3 at n >= 256; with ds's
+    2^-9 that stays under 2e-2."""
+    from sparseforge_amd import llama
+
+    S, H, D = 512, 2, 64
+    g = torch.Generator(device=cuda_device).manual_seed(2)
+    q, k = (torch.randn(1, S, H, D, generator=g, device=cuda_device) * 0.05 for _ in range(2))
+    v = 100.0 + torch.randn(1, S, H, D, generator=g, device=cuda_device)
+    q, k, v = (t.to(torch.bfloat16).requires_grad_(True) for t in (q, k, v))
+    go = torch.randn(1, S, H * D, generator=g, device=cuda_device).to(torch.bfloat16)
+    go[:, :256] = 0
+    cos, sin = torch.ones(S, D, device=cuda_device), torch.zeros(S, D, device=cuda_device)
+    o = llama.causal_attention(q, k, v, cos, sin)
+    dq, dk, _ = torch.autograd.grad(o, (q, k, v), go)
+    _, rg = _ref(q, k, v, cos, sin, go)
+    for a, b in ((dq, rg[0]), (dk, rg[1])):
+        assert float((a.double() - b.double()).norm() / b.double().norm()) < 2e-2
