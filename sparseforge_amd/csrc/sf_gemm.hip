@@ -1841,7 +1841,7 @@ extern "C" size_t sf_gemm_workspace_size(const sf_gemm_desc* d) {
   if (!d || d->M <= 0 || d->N <= 0 || d->K1 <= 0) return 0;
   if (d->dtype != SF_DTYPE_BF16 && d->dtype != SF_DTYPE_F32) return 0;
   if (skinny_ok(d)) return gemm_skinny_workspace(d->M, d->N, d->K1, d->a_layout, d->b_layout);
-  if (f32_dense(d)) return gemm_f32_workspace(d->M, d->N, d->K1);
+  if (f32_dense(d)) return gemm_f32_workspace(d->M, d->N, d->K1, d->a_layout);
   const int big = choose_splits(d);
   int sp = mid_dense(d) ? gemm_mid_splits(d->M, d->N, d->K1, d->c_blocks ? 1 : kMidMaxSplits, big) : 0;
   if (sp == 0) sp = big;

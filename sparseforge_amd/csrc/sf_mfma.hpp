@@ -110,7 +110,8 @@ struct GemmArgs {
   int64_t tiles_m, tiles_n;
   int splits;            // K splits (1: the kernel writes C itself)
   int64_t split_stages;  // segment-1 stages per split
-  float* partial;        // splits > 1: [splits][M][N] f32 partial sums
+  int64_t run_stages;    // f32 kernels: stages summed in one chain
+  float* partial;        // splits > 1 (or a split in several runs): [splits][M][N] f32 partial sums
   // block-sparse-16 B1 (B layouts 2 / 3): B1 is the blocks array, b_map its block map
   const int32_t* b_map;
   int64_t b_map_rows, b_map_cols;
@@ -260,7 +261,7 @@ int gemm_mid_splits(int64_t M, int64_t N, int64_t K, int max_splits, int big_spl
 int launch_gemm_mid(GemmArgs g, int a_layout, int b_layout, int splits, void* workspace, hipStream_t st);
 
 // The f32 product of dense, unmasked operands (sf_gemm_f32.hip): its workspace for K-split partials, and the launch.
-size_t gemm_f32_workspace(int64_t M, int64_t N, int64_t K);
+size_t gemm_f32_workspace(int64_t M, int64_t N, int64_t K, int a_layout);
 int launch_gemm_f32(GemmArgs g, int a_layout, int b_layout, void* workspace, size_t workspace_bytes, hipStream_t st);
 
 // y [N tokens, M out] = x W^T (+ A2/B2 low-rank term, + bias), W packed 2:4.

@@ -50,3 +50,26 @@ def test_segment_bias_mask_accumulate(cuda_device, M, N, K, R):
     assert gemm_err(got, prod + C.double(), torch.float32) <= 1.0
     for cap in (1, 2):  # fewer splits than planned: the workspace a caller gives
         assert gemm_err(lin.mm_nt(A, B, max_splits=cap, **kw), prod, torch.float32) <= 1.0
+
+
+@pytest.mark.parametrize("layout,M,N,K,pieces", [
+    ("nn", 8168, 768, 3072, 3), ("nt", 3312, 312, 632, 2), ("nn", 204, 3956, 804, 3), ("tn", 1024, 4096, 4096, 4),
+    ("nt", 1384, 1308, 1896, 7), ("nt", 2692, 560, 516, 2)])
+def test_error_of_the_sums(cuda_device, layout, M, N, K, pieces):
+    """K is summed in pieces (runs or splits), so that the rounding of a chain of adds stays that of its length: each of
+    n adds (two k each) of a random walk rounds by up to 2^-24 of a partial sum that has grown to sqrt(j / n) of the
+    result, 2^-24 sqrt(n / 6) in all (rms); 15 % for the sums of the pieces."""
+    from sparseforge_amd import linear as lin
+
+    g = torch.Generator(device=cuda_device).manual_seed(K)
+    A = _mk(g, cuda_device, *((K, M) if layout == "tn" else (M, K)))
+    B = _mk(g, cuda_device, *((N, K) if layout == "nt" else (K, N)))
+    a = A.double().t() if layout == "tn" else A.double()
+    b = B.double().t() if layout == "nt" else B.double()
+    ref = a.contiguous() @ b.contiguous()
+    err = float((getattr(lin, "mm_" + layout)(A, B).double() - ref).norm() / ref.norm())
+    assert err < 1.15 * 2.0 ** -24 * (K / pieces / 2 / 6) ** 0.5 + 2.0 ** -25, err
+    z, S = _mk(g, cuda_device, M, 20), _mk(g, cuda_device, N, 20)
+    if layout == "nt":  # a second segment after the last run
+        got = lin.mm_nt(A, B, A2=z, B2=S, K2=20)
+        assert gemm_err(got, ref + z.double() @ S.double().t(), torch.float32) <= 1.0
