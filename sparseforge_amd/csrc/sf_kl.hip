@@ -416,8 +416,11 @@ bool kl_vec_ok(std::initializer_list<const void*> ptrs) {
   return true;
 }
 // Rows up to one per CU leave too little in flight at 256 threads: 1024 threads a row (183 x 128256 bf16 forward 38 ->
-// 31 us, backward 47 -> 31; 76 x 32000 f32 15 and 16 -> 15 and 11).  600 rows are better at 256 (32 against 47 us).
-constexpr int64_t kKlFewRows = 257;
+// 31 us, backward 47 -> 31; 76 x 32000 f32 backward 16 -> 11).  600 rows are better at 256 (32 against 47 us).  The
+// forward's merge over 16 waves costs 1 to 2 us, which only rows of kKlWideBytes and more win back (256 and 1024
+// threads, 256 rows: 8192 bf16 9.1 and 11.2 us, 34968 bf16 16.9 and 18.1, 50257 bf16 21.1 and 19.8, 128256 bf16 41.7 and
+// 37.4); the backward has no merge.
+constexpr int64_t kKlFewRows = 257, kKlWideBytes = 96 << 10;
 // launch(data type, vector path, odd vocabulary) with the three as constants.
 template <typename F>
 void kl_dispatch(int dtype, bool vec, bool odd, F&& launch) {
@@ -465,10 +468,11 @@ extern "C" int sf_kl_forward(const void* student, const void* teacher, int dtype
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 grid(static_cast<unsigned>(rows));
   const bool odd = vocab % 8 != 0;
+  const bool wide = rows < kKlFewRows && vocab * (dtype == SF_DTYPE_F32 ? 4 : 2) >= kKlWideBytes;
   auto launch = [&](auto dt, auto v, auto o) {
     constexpr int DT = decltype(dt)::value;
     constexpr bool V = decltype(v)::value, ODD = decltype(o)::value;
-    if (rows < kKlFewRows)
+    if (wide)
       kl_rows_kernel<DT, V, ODD, 1024><<<grid, 1024, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_kl, row_nan);
     else
       kl_rows_kernel<DT, V, ODD, 256><<<grid, 256, 0, st>>>(student, teacher, vocab, inv_t, row_lse, row_kl, row_nan);

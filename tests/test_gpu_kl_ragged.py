@@ -39,3 +39,11 @@ def test_ragged_vocabulary(cuda_device, rows, vocab, dtype, shift):
     else:
         np.testing.assert_allclose(got, want, rtol=2.0 ** -7, atol=1e-3 * big + 1e-12)
     assert got[-1, -1] == 0.0
+
+
+@pytest.mark.parametrize("rows,vocab,dtype", [(3, 49157, torch.bfloat16), (65, 49152, torch.bfloat16),
+                                              (65, 24581, torch.float32), (3, 24576, torch.float32)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_few_wide_rows(cuda_device, rows, vocab, dtype, shift):
+    """The forward's 1024 threads a row: few rows of 96 KiB and more."""
+    test_ragged_vocabulary(cuda_device, rows, vocab, dtype, shift)
