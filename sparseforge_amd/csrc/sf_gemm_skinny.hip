@@ -261,10 +261,8 @@ int launch_tiles(const SkPlan& p, const GemmArgs& g, hipStream_t st) {
 }  // namespace
 
 size_t gemm_skinny_workspace(int64_t M, int64_t N, int64_t K, int a_layout, int b_layout) {
-  // K is always split (over the waves at least), which callers read from a size above zero; split over waves alone it
-  // needs no memory, and the 256 bytes are never touched
   const int sp = skinny_plan(M, N, K, (M <= N ? b_layout : a_layout) == SF_LAYOUT_MN, kSkMaxSplits).splits;
-  return sp > 1 ? static_cast<size_t>(sp) * M * N * sizeof(float) : 256;
+  return sp > 1 ? static_cast<size_t>(sp) * M * N * sizeof(float) : 0;  // K split over the waves alone needs none
 }
 
 int launch_gemm_skinny(GemmArgs g, int a_layout, int b_layout, void* workspace, size_t workspace_bytes, hipStream_t st) {

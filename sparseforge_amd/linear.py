@@ -114,7 +114,7 @@ def gemm(M, N, A1, B1, K1, a_layout, b_layout, *, A2=None, B2=None, K2=0, bmask=
     if max_splits is not None and ws_bytes > max_splits * M * N * 4:  # fewer K splits (the big products only)
         ws_bytes = max_splits * M * N * 4 if max_splits > 1 else 0
     ws = None
-    if ws_bytes > 256:  # split-K scratch from torch's caching allocator (256: split over waves, none needed)
+    if ws_bytes:  # split-K scratch from torch's caching allocator; the library never allocates
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         d.workspace, d.workspace_bytes = ws.data_ptr(), ws_bytes
     with _prof.region("sf_gemm", 2.0 * M * N * (K1 + K2), "FLOP", dev):

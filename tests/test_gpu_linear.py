@@ -293,10 +293,12 @@ def test_gemm_split_k_skinny(cuda_device, dtype):
     x = torch.randn(T, IN, generator=g).to(dtype)
     P = torch.randn(R, IN, generator=g).to(dtype)
     dz = torch.randn(T, R, generator=g).to(dtype)
-    desc = L.GemmDesc()
-    desc.dtype, desc.M, desc.N, desc.K1 = L.dtype_code(x), T, R, IN
-    assert L.lib().sf_gemm_workspace_size(L.byref(desc)) > 0  # this shape splits
     assert gemm_err(lin.mm_nt(d(x), d(P)), x.double() @ P.double().t(), dtype) <= 1.0
+    xs, Ps = torch.randn(T // 4, 8 * IN, generator=g).to(dtype), torch.randn(R, 8 * IN, generator=g).to(dtype)
+    desc = L.GemmDesc()
+    desc.dtype, desc.M, desc.N, desc.K1 = L.dtype_code(xs), T // 4, R, 8 * IN
+    assert L.lib().sf_gemm_workspace_size(L.byref(desc)) >= 2 * (T // 4) * R * 4  # this shape splits over workgroups
+    assert gemm_err(lin.mm_nt(d(xs), d(Ps)), xs.double() @ Ps.double().t(), dtype) <= 1.0
     assert gemm_err(lin.mm_tn(d(dz), d(x)), dz.double().t() @ x.double(), dtype) <= 1.0
     # second segment + bias on the last split, then accumulate into an existing C
     W = torch.randn(OUT, IN, generator=g).to(dtype)
