@@ -36,8 +36,7 @@ def _vec(dtype: torch.dtype) -> int:
 
 
 def gemm(M, N, A1, B1, K1, a_layout, b_layout, *, A2=None, B2=None, K2=0, bmask=None, bscale=1.0, bias=None,
-         emask=None, dw=None, decay=0.0, out=None, out_dtype=None, accumulate=False, bmask_t=None,
-         max_splits=None) -> torch.Tensor:
+         emask=None, dw=None, decay=0.0, out=None, out_dtype=None, accumulate=False, bmask_t=None) -> torch.Tensor:
     """C[M, N] = A1 . B1'^T (+ A2 . B2^T) on the device.
 
     a_layout: L.LAYOUT_K (A1 is [M, K]) or L.LAYOUT_MN (A1 is [K, M]);
@@ -111,8 +110,6 @@ def gemm(M, N, A1, B1, K1, a_layout, b_layout, *, A2=None, B2=None, K2=0, bmask=
         d.accumulate = 1
     ref, lib = ctypes.byref(d), L.lib()
     ws_bytes = lib.sf_gemm_workspace_size(ref)
-    if max_splits is not None and ws_bytes > max_splits * M * N * 4:  # fewer K splits (the big products only)
-        ws_bytes = max_splits * M * N * 4 if max_splits > 1 else 0
     ws = None
     if ws_bytes:  # split-K scratch from torch's caching allocator; the library never allocates
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)

@@ -1,4 +1,5 @@
 """pytest configuration: the `gpu` marker and shared fixtures."""
+import contextlib
 import os
 import sys
 
@@ -22,6 +23,28 @@ def load_golden(name: str) -> dict:
 
 
 BF16_ULP = 2.0 ** -7  # one bf16 ulp, relative to the value, at most
+
+
+@contextlib.contextmanager
+def gemm_workspace(splits):
+    """Products in the block get a workspace for at most `splits` K splits' partials (1: none; None: what they ask
+    for), as a C caller may give."""
+    from sparseforge_amd import _lib as L
+
+    lib = L.lib()
+    full = lib.sf_gemm_workspace_size
+
+    def size(ref):
+        d = ref._obj
+        room = splits * d.M * d.N * 4 if splits > 1 else 0
+        return min(full(ref), room)
+
+    if splits is not None:
+        lib.sf_gemm_workspace_size = size
+    try:
+        yield
+    finally:
+        lib.sf_gemm_workspace_size = full
 
 
 def gemm_err(got, ref, dtype, extra=None) -> float:

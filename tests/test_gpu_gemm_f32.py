@@ -4,7 +4,7 @@ of K terms is off by about sqrt(K) 2^-24 of the terms' scale, K at most 8168 her
 import pytest
 import torch
 
-from conftest import gemm_err
+from conftest import gemm_err, gemm_workspace
 
 pytestmark = pytest.mark.gpu
 
@@ -49,7 +49,8 @@ def test_segment_bias_mask_accumulate(cuda_device, M, N, K, R):
     got = lin.mm_nt(A, B, out=C.clone(), accumulate=True, **kw)
     assert gemm_err(got, prod + C.double(), torch.float32) <= 1.0
     for cap in (1, 2):  # fewer splits than planned: the workspace a caller gives
-        assert gemm_err(lin.mm_nt(A, B, max_splits=cap, **kw), prod, torch.float32) <= 1.0
+        with gemm_workspace(cap):
+            assert gemm_err(lin.mm_nt(A, B, **kw), prod, torch.float32) <= 1.0
 
 
 @pytest.mark.parametrize("layout,M,N,K,pieces", [

@@ -4,7 +4,7 @@ of the same operands (conftest.gemm_err)."""
 import pytest
 import torch
 
-from conftest import bias_slack, gemm_err
+from conftest import bias_slack, gemm_err, gemm_workspace
 
 pytestmark = pytest.mark.gpu
 
@@ -28,7 +28,8 @@ def test_layouts(cuda_device, M, N, K, layout):
     b = B.double().t() if layout == "nt" else B.double()
     ref = a @ b
     for cap in (None, 1, 2):
-        assert gemm_err(getattr(lin, "mm_" + layout)(A, B, max_splits=cap), ref, torch.bfloat16) <= 1.0
+        with gemm_workspace(cap):
+            assert gemm_err(getattr(lin, "mm_" + layout)(A, B), ref, torch.bfloat16) <= 1.0
 
 
 @pytest.mark.parametrize("M,N,K,R", [(80, 96, 128, 8), (1000, 264, 520, 72), (200, 2048, 4096, 64),
