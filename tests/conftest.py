@@ -47,6 +47,19 @@ def gemm_workspace(splits):
         lib.sf_gemm_workspace_size = full
 
 
+def gemm_splits(dtype, M, N, K) -> int:
+    """K splits over workgroups that the product A [M, K] B [N, K]^T asks a workspace for."""
+    import ctypes
+
+    import torch
+
+    from sparseforge_amd import _lib as L
+
+    d = L.GemmDesc()
+    d.dtype, d.M, d.N, d.K1 = int(dtype == torch.bfloat16), M, N, K
+    return L.lib().sf_gemm_workspace_size(ctypes.byref(d)) // (M * N * 4)
+
+
 def gemm_err(got, ref, dtype, extra=None) -> float:
     """Largest ratio of |got - ref| to the elementwise bar of a product accumulated in float32 and stored
     in `dtype`, against a float64 product of the same (already rounded) operands; <= 1 passes.

@@ -58,7 +58,7 @@ def test_large_scores_and_nan(cuda_device):
     o = llama.causal_attention(q, k, v, cos, sin)
     ro, _ = _ref(q, k, v, cos, sin, go)
     assert torch.isfinite(o).all()
-    assert float((o.double() - ro).norm() / ro.norm()) < 1e-2
+    assert float((o.double() - ro.detach()).norm() / ro.detach().norm()) < 1e-2
     v2 = v.clone()
     v2[0, 100, 1, 3] = float("nan")
     o2 = llama.causal_attention(q, k, v2, cos, sin).view(S, 2, D)
@@ -87,7 +87,8 @@ def test_double_backward_takes_the_materialised_path(cuda_device):
 
 
 def test_calls_outside_the_fused_path(cuda_device):
-    """float32, another head size and unaligned operands run the materialised path as before."""
+    """float32 and another head size run the materialised path, which refuses unaligned operands; the fused path takes
+    rows up to the softmax passes' longest."""
     from sparseforge_amd import llama
 
     for D, dt in ((64, torch.float32), (32, torch.bfloat16), (96, torch.bfloat16)):
@@ -96,6 +97,34 @@ def test_calls_outside_the_fused_path(cuda_device):
         assert not llama._fused_attention_takes(q, k, v, cos, sin)
         assert torch.equal(llama.causal_attention(q, k, v, cos, sin),
                            llama._causal_attention_device(q, k, v, cos, sin))
+    cos, sin = llama.rotary_tables(40, 64, 10000.0, cuda_device)
+    for which in range(3):  # one operand 2 bytes off a 16-byte boundary
+        qkv = [torch.randn(1, 40, 2, 64, device=cuda_device).to(torch.bfloat16) for _ in range(3)]
+        flat = torch.empty(40 * 2 * 64 + 1, dtype=torch.bfloat16, device=cuda_device)[1:]
+        qkv[which] = flat.view(1, 40, 2, 64).copy_(qkv[which])
+        assert not llama._fused_attention_takes(*qkv, cos, sin)
+        with pytest.raises(ValueError, match="aligned"):
+            llama.causal_attention(*qkv, cos, sin)
+    for S in (4096, 4097):
+        q = torch.empty(1, S, 1, 64, dtype=torch.bfloat16, device=cuda_device)
+        t = torch.empty(S, 64, device=cuda_device)
+        assert llama._fused_attention_takes(q, q, q, t, t) == (S <= llama.FUSED_MAX_S == 4096)
+
+
+def test_unaligned_and_strided_gradient(cuda_device):
+    """An upstream gradient 2 bytes off a boundary, or strided, gives the aligned one's gradients."""
+    from sparseforge_amd import llama
+
+    S, H, D = 70, 2, 64
+    q, k, v = (torch.randn(1, S, H, D, device=cuda_device).to(torch.bfloat16).requires_grad_(True) for _ in range(3))
+    cos, sin = llama.rotary_tables(S, D, 10000.0, cuda_device)
+    go = torch.randn(1, S, H * D, device=cuda_device).to(torch.bfloat16)
+    want = torch.autograd.grad(llama.causal_attention(q, k, v, cos, sin), (q, k, v), go)
+    off = torch.empty(go.numel() + 1, dtype=go.dtype, device=cuda_device)[1:].view_as(go).copy_(go)
+    strided = go.transpose(1, 2).contiguous().transpose(1, 2)
+    for g in (off, strided):
+        got = torch.autograd.grad(llama.causal_attention(q, k, v, cos, sin), (q, k, v), g)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
 @pytest.mark.parametrize("D", [64, 128])

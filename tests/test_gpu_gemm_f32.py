@@ -4,7 +4,7 @@ of K terms is off by about sqrt(K) 2^-24 of the terms' scale, K at most 8168 her
 import pytest
 import torch
 
-from conftest import gemm_err, gemm_workspace
+from conftest import gemm_err, gemm_splits, gemm_workspace
 
 pytestmark = pytest.mark.gpu
 
@@ -32,10 +32,12 @@ def test_layouts(cuda_device, M, N, K, layout):
     assert gemm_err(got, a @ b, torch.float32) <= 1.0
 
 
-@pytest.mark.parametrize("M,N,K,R", [(64, 96, 128, 4), (1000, 260, 516, 20), (48, 32, 8192, 64)])
+@pytest.mark.parametrize("M,N,K,R", [(64, 96, 128, 4), (1000, 260, 516, 20), (48, 32, 8192, 64), (1000, 704, 1952, 20)])
 def test_segment_bias_mask_accumulate(cuda_device, M, N, K, R):
     from sparseforge_amd import linear as lin
 
+    if (M, N) == (1000, 704):  # the split-K reduce of four columns a thread takes its epilogue from 2^19 outputs on
+        assert gemm_splits(torch.float32, M, N, K) > 1
     g = torch.Generator(device=cuda_device).manual_seed(M)
     A, B = _mk(g, cuda_device, M, K), _mk(g, cuda_device, N, K)
     z, S, bias = _mk(g, cuda_device, M, R), _mk(g, cuda_device, N, R), _mk(g, cuda_device, N)

@@ -4,7 +4,7 @@ of the same operands (conftest.gemm_err)."""
 import pytest
 import torch
 
-from conftest import bias_slack, gemm_err, gemm_workspace
+from conftest import bias_slack, gemm_err, gemm_splits, gemm_workspace
 
 pytestmark = pytest.mark.gpu
 
@@ -32,11 +32,13 @@ def test_layouts(cuda_device, M, N, K, layout):
             assert gemm_err(getattr(lin, "mm_" + layout)(A, B), ref, torch.bfloat16) <= 1.0
 
 
-@pytest.mark.parametrize("M,N,K,R", [(80, 96, 128, 8), (1000, 264, 520, 72), (200, 2048, 4096, 64),
+@pytest.mark.parametrize("M,N,K,R", [(80, 96, 128, 8), (1000, 264, 520, 72), (200, 2048, 4096, 64), (1000, 704, 1952, 72),
                                      (5632, 2048, 1032, 64)])  # the last on 256 x 256 tiles
 def test_segment_bias_mask_accumulate(cuda_device, M, N, K, R):
     from sparseforge_amd import linear as lin
 
+    if (M, N) == (1000, 704):  # the split-K reduce of four columns a thread takes its epilogue from 2^19 outputs on
+        assert gemm_splits(torch.bfloat16, M, N, K) > 1
     g = torch.Generator(device=cuda_device).manual_seed(M)
     A, B, z, S = (_mk(g, cuda_device, *s) for s in ((M, K), (N, K), (M, R), (N, R)))
     bias, C, W = _mk(g, cuda_device, N), _mk(g, cuda_device, M, N), _mk(g, cuda_device, M, N)

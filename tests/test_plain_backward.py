@@ -1,8 +1,14 @@
-"""Which backward passes run the gradient Functions' forwards directly: only those that nothing looks into."""
+"""Which backward passes run the gradient Functions' forwards directly: only those that nothing looks into; and that
+the package's gradient Functions can be run so."""
+import ast
+import inspect
+import textwrap
+
 import pytest
 import torch
 from torch.autograd import forward_ad
 
+from sparseforge_amd import distill, linear, llama
 from sparseforge_amd.linear import apply_in_backward
 
 
@@ -38,3 +44,25 @@ def test_forward_mode_is_refused_not_dropped():
 def test_vmap_is_refused():
     with torch.no_grad(), pytest.raises(RuntimeError):
         torch.func.vmap(lambda x: apply_in_backward(_Twice, x))(torch.ones(2, 3))
+
+
+GRADIENTS = [linear._MaskedLinearBackward, distill._KLGrad, llama._RMSNormGrad, llama._CausalSoftmaxGrad,
+             llama._SwiGLUGrad]
+
+
+def test_every_function_run_directly_is_listed():
+    used = set()
+    for module in (linear, distill, llama):
+        for node in ast.walk(ast.parse(inspect.getsource(module))):
+            if isinstance(node, ast.Call) and getattr(node.func, "id", "") == "apply_in_backward":
+                used.add(node.args[0].id)
+    assert used == {f.__name__ for f in GRADIENTS}
+
+
+@pytest.mark.parametrize("fn", GRADIENTS, ids=lambda f: f.__name__)
+def test_forward_asks_its_ctx_for_no_more_than_the_stand_in_has(fn):
+    """forward() may set attributes and call what _Unrecorded has; needs_input_grad and the like would be missing."""
+    tree = ast.parse(textwrap.dedent(inspect.getsource(fn.forward)))
+    loads = {n.attr for n in ast.walk(tree) if isinstance(n, ast.Attribute) and isinstance(n.ctx, ast.Load)
+             and isinstance(n.value, ast.Name) and n.value.id == "ctx"}
+    assert loads <= {name for name in vars(linear._Unrecorded) if not name.startswith("__")}
