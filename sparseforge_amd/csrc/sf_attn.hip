@@ -30,14 +30,17 @@
 // and sums of the two half-waves.
 //
 // A workgroup is 4 waves of 32 queries (or keys); tiles of 64 keys (or queries)
-// are loaded into registers one tile ahead and then into LDS.  Bound by the
-// softmax's VALU work (exp2 at a quarter rate: about 1000 clocks per 32 x 64 tile
-// against 512 of MFMA), so two or more workgroups share a CU.  The blocks of one
-// (batch, head) run on one XCD and share its keys and values in that L2; long
-// rows go first.
-// Measured at 2 x 2048 tokens, 32 heads of 64, causal: rotation 13 us, forward 72,
-// delta 9, dk / dv 144, dq 106, the whole call with its gradients 347 us; the
-// materialised products and softmax passes 1367 us.
+// are loaded into registers one tile ahead and then into LDS.  Heads of 64: 53 KB of
+// LDS, three workgroups a CU (dk / dv two, by its registers), and the softmax's VALU
+// work (exp2 at a quarter rate: about 1000 clocks per 32 x 64 tile against 512 of
+// MFMA) runs beside the MFMAs and LDS reads of the others.  Heads of 128: 86 KB, one
+// workgroup a CU, so nothing but its own four waves covers a tile's latencies.  The
+// blocks of one (batch, head) run on one XCD and share its keys and values in that
+// L2; long rows go first.
+// Measured, causal, us: rotation / forward / delta / dk, dv / dq:
+//   2 x 2048 tokens, 32 heads of 64    12 / 77 / 10 / 150 / 107, the call with its
+//     gradients 340; the materialised products and softmax passes 1367
+//   1 x 2048 tokens, 32 heads of 128   12 / 107 / 9 / 158 / 144
 #include <type_traits>
 
 #include "sf_mfma.hpp"
@@ -73,6 +76,9 @@ struct AttnArgs {
 // banks and the transposed reads of 4 rows x 64 bytes overlap in 4 words only.
 template <int D>
 constexpr int at_pitch() { return D == 64 ? 208 : 336; }
+// Workgroups a CU that the registers are limited for (LDS: three with heads of 64, one with heads of 128).
+template <int D>
+constexpr int at_wgs() { return D == 64 ? 2 : 1; }
 
 __host__ __device__ __forceinline__ float* at_flag(const AttnArgs& a) { return a.stats + 3 * (int64_t)a.BH * a.S; }
 
@@ -263,7 +269,7 @@ __device__ __forceinline__ void store_rows_f32(float* t, const AttnArgs& a, int 
 // Forward: 128 queries of one (batch, head).
 // ---------------------------------------------------------------------------
 template <int D>
-__global__ void __launch_bounds__(256, 2) attn_fwd_kernel(AttnArgs a, int nb) {
+__global__ void __launch_bounds__(256, at_wgs<D>()) attn_fwd_kernel(AttnArgs a, int nb) {
   __shared__ __align__(16) unsigned char ks[2][kAtTile * at_pitch<D>()];
   __shared__ __align__(16) unsigned char vs[2][kAtTile * at_pitch<D>()];
   int bh, blk;
@@ -398,7 +404,7 @@ __global__ void __launch_bounds__(256) attn_delta_kernel(AttnArgs a, int64_t wor
 // dq: 128 queries of one (batch, head), tiles of 64 keys.
 // ---------------------------------------------------------------------------
 template <int D>
-__global__ void __launch_bounds__(256, 2) attn_dq_kernel(AttnArgs a, int nb) {
+__global__ void __launch_bounds__(256, at_wgs<D>()) attn_dq_kernel(AttnArgs a, int nb) {
   __shared__ __align__(16) unsigned char ks[2][kAtTile * at_pitch<D>()];
   __shared__ __align__(16) unsigned char vs[2][kAtTile * at_pitch<D>()];
   int bh, blk;
@@ -571,7 +577,7 @@ __device__ __forceinline__ void attn_dkv_block(const AttnArgs& a, int nb, DkvLds
 }
 
 template <int D>
-__global__ void __launch_bounds__(256, D == 64 ? 2 : 1) attn_dkv_kernel(AttnArgs a, int nb) {
+__global__ void __launch_bounds__(256, at_wgs<D>()) attn_dkv_kernel(AttnArgs a, int nb) {
   __shared__ __align__(16) DkvLds<D> sm;
   if (__builtin_expect(*at_flag(a) != 0.0f, 0))
     attn_dkv_block<D, true>(a, nb, sm);
