@@ -31,13 +31,6 @@ constexpr size_t sp_smem() {
   return stage > red ? stage : red;
 }
 
-// Orders a wave's LDS writes before its own later reads for the compiler (the hardware keeps the order).
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The low-rank term A2 . B2^T of a tile of RB * 32 outputs from m0 and NT * 32 tokens from n0 on the dense MFMA:
 // 16-k steps first, first + step, ... with both operands straight from memory (a few KiB per tile).
 template <int RB, int NT>

@@ -26,12 +26,6 @@ namespace {
 
 constexpr int kSkWaves = 8;
 
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // One operand's stage: NB * 32 rows x 64 k.  L = 0: 128-byte rows of 8 k-chunks, chunk XOR f(row) =
 // (row ^ row / 8) & 7.  L = 1: 64 k-rows of NB * 4 chunks; with 8 chunks, chunk XOR 4 ((k / 2) & 1), so the four
 // rows that a transposed read takes lie in different banks.

@@ -64,6 +64,13 @@ __device__ __forceinline__ V4 bload(Rsrc r, uint32_t voff, uint32_t soff) {
   return o;
 }
 
+// Orders a wave's LDS writes before its own later reads for the compiler (the hardware keeps the order).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __device__ __forceinline__ float load_elem(const void* p, int64_t i, int dtype) { return load_as_f32(p, i, dtype); }
 
 constexpr int kGroupM = 8;  // M-tiles per L2 band
