@@ -214,3 +214,38 @@ def test_delta_from_the_unrounded_output(cuda_device):
     _, rg = _ref(q, k, v, cos, sin, go)
     for a, b in ((dq, rg[0]), (dk, rg[1])):
         assert float((a.double() - b.double()).norm() / b.double().norm()) < 2e-2
+
+
+def test_graph_replays(cuda_device):
+    """A captured forward and backward, replayed on inputs whose scores run away, then do not, and again: the word that
+    selects the backward's body is written anew each time."""
+    from sparseforge_amd import llama
+
+    S, H, D = 130, 2, 64
+    cos, sin = llama.rotary_tables(S, D, 10000.0, cuda_device)
+    g = torch.Generator(device=cuda_device).manual_seed(9)
+    mk = lambda f: [(torch.randn(1, S, H, D, generator=g, device=cuda_device) * f).to(torch.bfloat16) for _ in range(3)]  # noqa: E731
+    q, k, v = (t.requires_grad_(True) for t in mk(1.0))
+    go = torch.randn(1, S, H * D, generator=g, device=cuda_device).to(torch.bfloat16)
+
+    def call():
+        o = llama.causal_attention(q, k, v, cos, sin)
+        return (o.detach(), *torch.autograd.grad(o, (q, k, v), go))
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = call()
+    for size in (1.0, 1e4, 2.0, 1e6):
+        with torch.no_grad():
+            for t, new in zip((q, k, v), mk(size)):
+                t.copy_(new)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [t.clone() for t in outs]
+        for a, b in zip(got, call()):
+            assert torch.isfinite(a).all() and torch.equal(a, b)
